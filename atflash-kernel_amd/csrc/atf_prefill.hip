@@ -417,6 +417,36 @@ __device__ __forceinline__ float exp_tiles(const f32x16 (&S)[4], bf16x8 (&Pf)[8]
   return lt;
 }
 
+// Block -> (sequence, q head, query tile), XCD-aware: block i runs on XCD i % 8
+// (were it not so, that would cost time, not results).  The units (query tile,
+// sequence, kv head), heaviest (last) tiles first, are dealt out one to an XCD in
+// turn, in alternating XCD order from one round of 8 units to the next
+// (serpentine), so that every XCD gets the same causal work; the q heads of a
+// unit are consecutive on its XCD and share its K/V tiles in that XCD's L2.
+// Where 8 divides into the kv heads or the other way round, an XCD so holds one
+// kv head (or a fixed few) of every second tile.
+//   Dealing out whole query tiles instead (all heads of a tile on one XCD, one
+// sequence after the other) left XCDs without work below 8 tiles a sequence,
+// whatever the batch: 8 x 700 tokens of 24 heads ran on 3 of 8 XCDs, 191 us
+// against 82 here; 1024 queries behind 32K keys (28 heads) on 4, 649 against
+// 531; 4 x 2048 tokens 237 against 172; 5000 tokens 197 against 187.  At 32K
+// tokens and up the two are within 1% (28 / 4 heads, windowed 128K 75.9 ms
+// against 75.6), 4% in favour of this one with 24 / 8 heads (68.6 against 65.9);
+// outputs bitwise equal.
+__device__ __forceinline__ bool prefill_block(const PrefillArgs& a, int bid, int& b, int& h, int& qt) {
+  const int xcd = bid & 7;
+  const int j = bid >> 3;
+  const int rnd = j / a.group;
+  const int unit = rnd * 8 + ((rnd & 1) ? 7 - xcd : xcd);
+  const int per_tile = a.batch * a.hkv;
+  const int qrank = unit / per_tile;
+  const int r = unit - qrank * per_tile;
+  b = r / a.hkv;
+  h = (r - b * a.hkv) * a.group + (j - rnd * a.group);
+  qt = a.n_qtiles - 1 - qrank;
+  return qt >= 0;
+}
+
 // kRaw selects how the softmax scale c = sm_scale * log2(e) is applied.
 //   false (RoPE at load): Q is rotated and multiplied by c in fp32 and rounded
 //         to bf16 once, so the MFMAs return scores in log2 units directly;
@@ -432,25 +462,8 @@ __global__ __launch_bounds__(kPfWaves * 64, 1) void prefill_kernel(PrefillArgs a
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
-  // XCD-aware block mapping: block i runs on XCD i % 8.  Each XCD walks the q
-  // heads of one q-tile in order (so the heads sharing a kv head share its K/V
-  // tiles in that XCD's L2), and the 8 XCDs take 8 neighbouring q-tiles, the
-  // heaviest (last) tiles first.  With a.xcd_alt the XCD order alternates from
-  // one round of 8 tiles to the next (serpentine), so that every XCD gets the
-  // same causal work over two rounds; with the same order in every round the
-  // first XCD takes the heaviest tile of every round (prefill_xcd_alternate
-  // decides per launch).
-  const int bid = blockIdx.x;
-  const int xcd = bid & 7;
-  const int j = bid >> 3;
-  const int per_b = a.n_qgroups * a.hq;
-  const int b = j / per_b;
-  const int jr = j - b * per_b;
-  const int h = jr % a.hq;
-  const int rnd = jr / a.hq;
-  const int qrank = rnd * 8 + ((rnd & a.xcd_alt & 1) ? 7 - xcd : xcd);
-  const int qt = a.n_qtiles - 1 - qrank;
-  if (qt < 0 || b >= a.batch) return;
+  int b, h, qt;
+  if (!prefill_block(a, blockIdx.x, b, h, qt)) return;
   const int kvh = h / a.group;
 
   const int lr0_wg = qt * kPfRowsWg;
@@ -786,8 +799,8 @@ __device__ __forceinline__ u32x4 probe_vec(uint32_t seed, bool unit) {
                probe_bf16x2(probe_hash(seed * 4 + 2), unit), probe_bf16x2(probe_hash(seed * 4 + 3), unit)};
 }
 
-// The prefill kernel's MFMA work with nothing else: the same grid, block
-// mapping, waves, tile-pair count per workgroup (causal, nk = nq, window OFF),
+// The prefill kernel's MFMA work with nothing else: the same grid
+// (heaviest tiles first, serpentine over the XCDs), waves, tile-pair count per workgroup (causal, nk = nq, window OFF),
 // LDS operand ring and stream order (PV of 8 pages then QK of 8 levels over
 // four 32-key blocks, 64 MFMAs per pair), s_setprio and the two barriers per
 // pair with the two wave groups one phase apart -- but no softmax, no K/V
@@ -797,7 +810,7 @@ __device__ __forceinline__ u32x4 probe_vec(uint32_t seed, bool unit) {
 // structure at the clock the part's power limit allows.  The accumulators are
 // kept live by an empty asm statement and one store per lane at the end.
 __global__ __launch_bounds__(kPfWaves * 64, 1) void prefill_mfma_probe_kernel(int nq, int hq, int n_qtiles,
-                                                                               int xcd_alt, float* sink) {
+                                                                               float* sink) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem_raw[];
   lds_u8* smem = (lds_u8*)(smem_raw);
   const int tid = threadIdx.x;
@@ -808,7 +821,7 @@ __global__ __launch_bounds__(kPfWaves * 64, 1) void prefill_mfma_probe_kernel(in
   const int j = bid >> 3;
   const int h = j % hq;
   const int rnd = j / hq;
-  const int qrank = rnd * 8 + ((rnd & xcd_alt & 1) ? 7 - xcd : xcd);  // prefill_kernel's order
+  const int qrank = rnd * 8 + ((rnd & 1) ? 7 - xcd : xcd);
   const int qt = n_qtiles - 1 - qrank;
   if (qt < 0) return;
   const int last_wg = min(nq, qt * kPfRowsWg + kPfRowsWg) - 1;
@@ -900,43 +913,16 @@ hipError_t ensure_lds_attribute() {
 }
 }  // namespace
 
-// Whether a launch takes the serpentine XCD order.  With the same order in
-// every round of 8 q-tiles, XCD x gets tiles n-1-x, n-9-x, ...: the first XCD
-// holds the heaviest tile of every round and finishes last.  Where that puts
-// the busiest XCD's causal work (the k-tiles of its workgroups) more than 1%
-// above the mean, the order alternates (same-box A/B, outputs bitwise equal:
-// Llama-3.2-3B shape single shot, 8K -9 to -11%, 32K -2 to -3.6%; Qwen2.5-7B
-// shape 32K in 8K chunks -1 to -1.5%; 128K single shot OFF -0.4 to -0.5%,
-// k=2 -0.2 to +0.1% over 11 to 15 interleaved repetitions).  Where
-// the tiles' work is nearly equal (a late chunk of a chunked prefill, whose
-// keys are mostly the cached prefix) the plain order is kept: there the
-// serpentine one measured 0 to 1% slower (Qwen2.5-7B shape, 256K in 8K chunks).
-int prefill_xcd_alternate(int n_qtiles, int nq, int nk, int q_offset) {
-  const int n_ktiles = (nk + kPfTileN - 1) / kPfTileN;
-  double tot[8] = {};
-  for (int qrank = 0; qrank < n_qtiles; ++qrank) {
-    const int qt = n_qtiles - 1 - qrank;
-    const int last = q_offset + std::min(nq, (qt + 1) * kPfRowsWg) - 1;
-    tot[qrank & 7] += std::min(n_ktiles, last / kPfTileN + 1);
-  }
-  double mx = 0.0, sum = 0.0;
-  for (double t : tot) {
-    mx = std::max(mx, t);
-    sum += t;
-  }
-  return (sum > 0.0 && 8.0 * mx > 1.01 * sum) ? 1 : 0;
-}
-
 hipError_t launch_prefill(const PrefillArgs& a, hipStream_t s) {
   if (a.nq <= 0 || a.batch <= 0) return hipSuccess;
   if (hipError_t e = ensure_lds_attribute(); e != hipSuccess) return e;
-  const int blocks = a.batch * a.n_qgroups * a.hq * 8;
-  PrefillArgs k = a;
-  k.xcd_alt = prefill_xcd_alternate(a.n_qtiles, a.nq, a.nk, a.q_offset);
+  const int64_t units = static_cast<int64_t>(a.n_qtiles) * a.batch * a.hkv;
+  const int64_t blocks = (units + 7) / 8 * 8 * a.group;
+  if (blocks > INT32_MAX) return hipErrorInvalidConfiguration;
   if (a.rope_cs != nullptr)
-    hipLaunchKernelGGL(prefill_kernel<false>, dim3(blocks), dim3(kPfWaves * 64), kPfLdsTotal, s, k);
+    hipLaunchKernelGGL(prefill_kernel<false>, dim3(blocks), dim3(kPfWaves * 64), kPfLdsTotal, s, a);
   else
-    hipLaunchKernelGGL(prefill_kernel<true>, dim3(blocks), dim3(kPfWaves * 64), kPfLdsTotal, s, k);
+    hipLaunchKernelGGL(prefill_kernel<true>, dim3(blocks), dim3(kPfWaves * 64), kPfLdsTotal, s, a);
   return hipGetLastError();
 }
 
@@ -945,8 +931,7 @@ hipError_t launch_prefill_mfma_probe(float* sink, int nq, int hq, hipStream_t s)
   if (hipError_t e = ensure_lds_attribute(); e != hipSuccess) return e;
   const int n_qtiles = (nq + kPfRowsWg - 1) / kPfRowsWg;
   const int blocks = ((n_qtiles + 7) / 8) * hq * 8;
-  hipLaunchKernelGGL(prefill_mfma_probe_kernel, dim3(blocks), dim3(kPfWaves * 64), kPfLdsTotal, s, nq, hq, n_qtiles,
-                     prefill_xcd_alternate(n_qtiles, nq, nq, 0), sink);
+  hipLaunchKernelGGL(prefill_mfma_probe_kernel, dim3(blocks), dim3(kPfWaves * 64), kPfLdsTotal, s, nq, hq, n_qtiles, sink);
   return hipGetLastError();
 }
 
