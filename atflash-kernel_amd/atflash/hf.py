@@ -38,9 +38,10 @@ call consumed (another attention implementation read the layer, or the key
 reached the hook as a copy) makes the next call on that layer raise instead of
 attending to the chunk only, and unregister() closes the caches of the hook it
 removes.  With any other cache (HF's DynamicCache passes the whole history as
-key/value) the hook packs that history into a temporary paged cache per call --
-correct, but it rewrites the whole context every call (a warning says so once
-per hook), so long contexts should use PagedCache.
+key/value) a prefill packs that history into a temporary paged cache per call and
+a decode reads it in place -- correct, but every call goes over the whole context
+again, rotating its keys, and a decode's window saves less than on pages (a
+warning says so once per hook), so long contexts should use PagedCache.
 """
 import warnings
 import weakref
@@ -327,16 +328,15 @@ class WindowAttention:
         # any other cache: key/value hold the whole history [b, hkv, S, d]
         if not self._warned_repack and S > 4096:
             self._warned_repack = True
-            warnings.warn(f"atflash.hf: a plain KV cache ({S} tokens) is re-packed into a temporary paged cache on "
-                          "every attention call (the cache writer over the whole history, then the kernel); use "
+            warnings.warn(f"atflash.hf: a plain KV cache ({S} tokens) is gone over again on every attention call (a "
+                          "prefill re-packs it into a temporary paged cache, a decode rotates its keys anew); use "
                           "hook.new_cache(...) as past_key_values to attend on persistent pages", RuntimeWarning,
                           stacklevel=2)
         rt = self.rope_table(S, query.device)
         if L == 1:
-            kvc, table = I.pack_kv(key.transpose(1, 2), value.transpose(1, 2), rope=rt)
-            seq = torch.full((b,), S, dtype=torch.int32, device=query.device)
             zhi = self.window.decode_zhi8 if windowed else None
-            o = ops.decode_paged(query[:, :, 0, :], kvc, table, seq, S, zhi, scale, rt, 0)
+            o = I.decode_contiguous(query[:, :, 0, :], key.transpose(1, 2), value.transpose(1, 2), zhi, scale, rt,
+                                    _lib.LAYOUT_HALF_SPLIT)
             return o.view(b, 1, hq, d), None
         zhi = self.window.prefill_zhi if windowed else None
         o, _ = I._flash_attn_fwd(query.transpose(1, 2), key.transpose(1, 2), value.transpose(1, 2), causal=True,

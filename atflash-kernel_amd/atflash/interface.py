@@ -13,11 +13,12 @@ paged    `prefill_paged` / `decode_paged` on a PagedKVCache, the serving path;
 
 Cost of the contiguous entry points: `_flash_attn_fwd` and
 `single_decode_with_kv_cache` take the whole history as contiguous k/v, like the
-reference's kernels, so every call first packs it into a fresh paged cache
+reference's kernels.  The prefill first packs it into a fresh paged cache
 (`pack_kv`: an allocation and the cache writer over all Nk tokens, about 124 us
-at 128K tokens x 4 kv heads) before the attention kernel.  A decode loop should
-keep a PagedKVCache (or atflash.hf.PagedCache) and call `decode_paged`, which
-writes each token once.
+at 128K tokens x 4 kv heads) before the attention kernel.  The decode reads the
+rows in place; its window then saves less than on pages, whose K is stored by
+wavelength, so a decode loop should keep a PagedKVCache (or atflash.hf.PagedCache)
+and call `decode_paged`.
 
 Differences from the reference that a caller sees:
   * prefill takes the 16-dim level table zhi; decode takes either the
@@ -95,21 +96,29 @@ def _flash_attn_fwd(q, k, v, causal=True, pack_gqa=None, atflash_window_zhi=None
 
 def single_decode_with_kv_cache(q, k, v, maybe_zhi=None, sm_scale=None, kv_layout="NHD", rope=None,
                                 layout="half_split"):
-    """One query token per q head against a contiguous KV (convenience path: the
-    KV is packed into a temporary paged cache first).  Returns o [Hq, 128] bf16.
+    """One query token per q head against a contiguous KV, read in place.
+    Returns o [Hq, 128] bf16.
     maybe_zhi: the level table (8 entries, page rule) or the FlashInfer port's
     per-slice table (16 entries, fiwin_common.zhi_slice_vec8, per-key rule)."""
     if kv_layout == "HND":
         k, v = k.transpose(0, 1), v.transpose(0, 1)
     elif kv_layout != "NHD":
         raise ValueError("kv_layout must be NHD or HND")
-    N = k.shape[0]
     scale = 1.0 / math.sqrt(q.shape[-1]) if sm_scale is None else float(sm_scale)
-    kv_cache, table = pack_kv(k.unsqueeze(0), v.unsqueeze(0), rope=rope, layout=layout)
-    seq = torch.tensor([N], dtype=torch.int32, device=q.device)
-    o = ops.decode_paged(q.unsqueeze(0), kv_cache, table, seq, N, _zhi_list(maybe_zhi, _DECODE_TABLES), scale,
-                         rope, _layout_id(layout))
-    return o[0]
+    return decode_contiguous(q.unsqueeze(0), k.unsqueeze(0), v.unsqueeze(0), _zhi_list(maybe_zhi, _DECODE_TABLES),
+                             scale, rope, _layout_id(layout))[0]
+
+
+def decode_contiguous(q, k, v, zhi, scale, rope, layout):
+    """Decode of q [B, Hq, 128] over contiguous-sequence k, v [B, N, Hkv, 128]:
+    in place, or packed into pages where the token strides are too long for that."""
+    o = ops.decode_rows(q, k, v, zhi, scale, rope, layout)
+    if o is None:
+        N = k.shape[1]
+        kv_cache, table = pack_kv(k, v, rope=rope, layout=layout)
+        seq = torch.full((k.shape[0],), N, dtype=torch.int32, device=q.device)
+        o = ops.decode_paged(q, kv_cache, table, seq, N, zhi, scale, rope, layout)
+    return o
 
 
 def prefill_paged(q, cache, page_table, nk, q_offset, zhi=None, sm_scale=None, rope=None, layout="half_split"):

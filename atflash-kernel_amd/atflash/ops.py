@@ -214,6 +214,46 @@ def decode_paged(q: torch.Tensor, kv_cache: torch.Tensor, page_table: torch.Tens
     return out
 
 
+# Longest token stride (elements) of the K and V rows atf_decode_rows_bf16 reads.
+_ROWS_MAX_STRIDE = 1 << 26
+
+
+def decode_rows(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, zhi, sm_scale: float,
+                rope_cs: Optional[torch.Tensor], layout: int) -> Optional[torch.Tensor]:
+    """Decode of q [B, Hq, 128] over contiguous-sequence k, v [B, N, Hkv, 128]
+    (strided views accepted) read in place; the query sits at position N - 1.
+    zhi as decode_paged's.  Returns out bf16 [B, Hq, 128], or None for token
+    strides past what the kernel addresses (the caller packs those into pages)."""
+    _need_gpu(q, k, v, rope_cs)
+    _need(k.dtype == torch.bfloat16 and v.dtype == torch.bfloat16, "k and v must be bf16")
+    ks = k.shape
+    _need(len(ks) == 4 and v.shape == ks and ks[3] == _lib.HEAD_DIM, "k and v must be [B, T, Hkv, 128] of equal shape")
+    kst, vst = k.stride(), v.stride()
+    _need(kst[3] == 1 and vst[3] == 1, "last dim of k and v must be contiguous")
+    qs = q.shape
+    _need(q.dtype == torch.bfloat16 and len(qs) == 3 and qs[2] == _lib.HEAD_DIM, "q must be bf16 [B, Hq, 128]")
+    q_sb, q_sh, q_sd = q.stride()
+    _need(q_sd == 1, "last dim of q must be contiguous")
+    _need(qs[0] == ks[0], "q and k must have the same batch")
+    if kst[1] > _ROWS_MAX_STRIDE or vst[1] > _ROWS_MAX_STRIDE:
+        return None
+    B, N, hkv, _ = ks
+    Hq = qs[1]
+    rope_cs, max_pos = _rope(rope_cs)
+    L = _lib.lib()
+    dev = q.device
+    stream = _lib.stream_of(dev)
+    ws = _decode_workspace(dev, stream, B, Hq, hkv, N, L)
+    out = torch.empty((B, Hq, _lib.HEAD_DIM), dtype=torch.bfloat16, device=dev)
+    n = 0 if zhi is None else len(zhi)
+    _lib.check(L.atf_decode_rows_bf16(
+        out.data_ptr(), Hq * _lib.HEAD_DIM, _lib.HEAD_DIM, q.data_ptr(), q_sb, q_sh,
+        k.data_ptr(), kst[0], kst[1], kst[2], v.data_ptr(), vst[0], vst[1], vst[2],
+        B, Hq, hkv, N, _table(zhi, n), n, float(sm_scale), _lib.ptr(rope_cs), max_pos, _layout(layout),
+        ws[0], ws[1], stream))
+    return out
+
+
 class DecodePlan:
     """A decode call prepared once and run many times (a serving loop's step).
 

@@ -238,29 +238,16 @@ size_t atf_decode_workspace_bytes(int batch, int num_q_heads, int num_kv_heads, 
 
 namespace {
 
-// Validation and argument packing shared by the two decode entry points
-// (everything except the workspace).
-int decode_prepare(void* out, int64_t o_sb, int64_t o_sh, const void* q, int64_t q_sb, int64_t q_sh,
-                   const void* kv_cache, int num_pages, const int32_t* page_table, int max_pages,
-                   const int32_t* seq_lens, int batch, int num_q_heads, int num_kv_heads, int max_seq_len,
-                   const int32_t* zhi, bool slice_table, float sm_scale, const float* rope_cs, int rope_max_pos,
-                   int layout, atf::DecodeArgs* a) {
-  if (!out || !q || !kv_cache || !page_table || !seq_lens)
-    return fail(ATF_ERR_INVALID, "null pointer argument");
-  if (num_q_heads <= 0 || num_kv_heads <= 0 || num_q_heads % num_kv_heads != 0)
-    return fail(ATF_ERR_INVALID, "num_q_heads (%d) must be a positive multiple of num_kv_heads (%d)", num_q_heads,
-                num_kv_heads);
-  if (num_q_heads / num_kv_heads > atf::kDecMaxGroup)
-    return fail(ATF_ERR_UNSUPPORTED, "GQA group %d > %d", num_q_heads / num_kv_heads, atf::kDecMaxGroup);
-  if (max_seq_len <= 0 || max_seq_len >= (1 << 24)) return fail(ATF_ERR_INVALID, "max_seq_len out of range");
-  if (num_pages <= 0 || max_pages <= 0 || static_cast<int64_t>(max_pages) * atf::kPage < max_seq_len)
-    return fail(ATF_ERR_INVALID, "page table too small for max_seq_len=%d (max_pages=%d)", max_seq_len, max_pages);
+// Validation and argument packing shared by the decode entry points
+// (everything except the keys and the workspace).
+int decode_prepare_query(void* out, int64_t o_sb, int64_t o_sh, const void* q, int64_t q_sb, int64_t q_sh, int batch,
+                         int num_q_heads, int num_kv_heads, int max_seq_len, const int32_t* zhi, bool slice_table,
+                         float sm_scale, const float* rope_cs, int rope_max_pos, int layout, atf::DecodeArgs* a) {
   if (!(sm_scale > 0.f) || !std::isfinite(sm_scale)) return fail(ATF_ERR_INVALID, "sm_scale must be positive");
   if (int r = check_layout(layout, rope_cs, rope_max_pos)) return r;
   if (rope_cs && max_seq_len > rope_max_pos)
     return fail(ATF_ERR_INVALID, "rope table has %d positions, need %d", rope_max_pos, max_seq_len);
-  if (!aligned(q, 16) || !aligned(out, 8) || !aligned(kv_cache, 16))
-    return fail(ATF_ERR_INVALID, "q and kv_cache must be 16-byte and out 8-byte aligned");
+  if (!aligned(q, 16) || !aligned(out, 8)) return fail(ATF_ERR_INVALID, "q must be 16-byte and out 8-byte aligned");
   if (q_sb % 8 || q_sh % 8) return fail(ATF_ERR_INVALID, "q strides must be multiples of 8 elements");
   if (o_sb % 4 || o_sh % 4) return fail(ATF_ERR_INVALID, "out strides must be multiples of 4 elements");
   if (int r = slice_table ? make_decode_table_slices(zhi, a)
@@ -272,11 +259,6 @@ int decode_prepare(void* out, int64_t o_sb, int64_t o_sh, const void* q, int64_t
   a->q = static_cast<const uint16_t*>(q);
   a->q_sb = q_sb;
   a->q_sh = q_sh;
-  a->kv_cache = static_cast<const uint16_t*>(kv_cache);
-  a->num_pages = num_pages;
-  a->page_table = page_table;
-  a->max_pages = max_pages;
-  a->seq_lens = seq_lens;
   a->max_seq_len = max_seq_len;
   a->batch = batch;
   a->hq = num_q_heads;
@@ -290,6 +272,47 @@ int decode_prepare(void* out, int64_t o_sb, int64_t o_sh, const void* q, int64_t
   a->out = static_cast<uint16_t*>(out);
   a->o_sb = o_sb;
   a->o_sh = o_sh;
+  return ATF_OK;
+}
+
+int check_decode_heads(int num_q_heads, int num_kv_heads, int max_seq_len) {
+  if (num_q_heads <= 0 || num_kv_heads <= 0 || num_q_heads % num_kv_heads != 0)
+    return fail(ATF_ERR_INVALID, "num_q_heads (%d) must be a positive multiple of num_kv_heads (%d)", num_q_heads,
+                num_kv_heads);
+  if (num_q_heads / num_kv_heads > atf::kDecMaxGroup)
+    return fail(ATF_ERR_UNSUPPORTED, "GQA group %d > %d", num_q_heads / num_kv_heads, atf::kDecMaxGroup);
+  if (max_seq_len <= 0 || max_seq_len >= (1 << 24)) return fail(ATF_ERR_INVALID, "max_seq_len out of range");
+  return ATF_OK;
+}
+
+int decode_prepare(void* out, int64_t o_sb, int64_t o_sh, const void* q, int64_t q_sb, int64_t q_sh,
+                   const void* kv_cache, int num_pages, const int32_t* page_table, int max_pages,
+                   const int32_t* seq_lens, int batch, int num_q_heads, int num_kv_heads, int max_seq_len,
+                   const int32_t* zhi, bool slice_table, float sm_scale, const float* rope_cs, int rope_max_pos,
+                   int layout, atf::DecodeArgs* a) {
+  if (!out || !q || !kv_cache || !page_table || !seq_lens)
+    return fail(ATF_ERR_INVALID, "null pointer argument");
+  if (int r = check_decode_heads(num_q_heads, num_kv_heads, max_seq_len)) return r;
+  if (num_pages <= 0 || max_pages <= 0 || static_cast<int64_t>(max_pages) * atf::kPage < max_seq_len)
+    return fail(ATF_ERR_INVALID, "page table too small for max_seq_len=%d (max_pages=%d)", max_seq_len, max_pages);
+  if (!aligned(kv_cache, 16)) return fail(ATF_ERR_INVALID, "kv_cache must be 16-byte aligned");
+  a->kv_cache = static_cast<const uint16_t*>(kv_cache);
+  a->num_pages = num_pages;
+  a->page_table = page_table;
+  a->max_pages = max_pages;
+  a->seq_lens = seq_lens;
+  return decode_prepare_query(out, o_sb, o_sh, q, q_sb, q_sh, batch, num_q_heads, num_kv_heads, max_seq_len, zhi,
+                              slice_table, sm_scale, rope_cs, rope_max_pos, layout, a);
+}
+
+// The caller's workspace -> the split partials' addresses.
+int set_workspace(void* workspace, size_t workspace_bytes, atf::DecodeArgs* a) {
+  const size_t need = partial_bytes(a->batch, a->hkv, a->n_splits);
+  if (need > 0 && (!workspace || workspace_bytes < need || !aligned(workspace, 16)))
+    return fail(ATF_ERR_WORKSPACE, "workspace of %zu bytes (16-byte aligned) required, got %zu", need,
+                workspace ? workspace_bytes : 0);
+  a->ws_ml = static_cast<float*>(workspace);
+  a->ws_o = need > 0 ? a->ws_ml + static_cast<size_t>(a->batch) * a->hkv * a->n_splits * atf::kDecMaxGroup * 2 : nullptr;
   return ATF_OK;
 }
 
@@ -311,13 +334,7 @@ int decode_with_workspace(void* out, int64_t o_sb, int64_t o_sh, const void* q, 
                              seq_lens, batch, num_q_heads, num_kv_heads, max_seq_len, zhi, slice_table, sm_scale,
                              rope_cs, rope_max_pos, layout, &a))
     return r;
-  const size_t need = partial_bytes(batch, num_kv_heads, a.n_splits);
-  if (need > 0 && (!workspace || workspace_bytes < need || !aligned(workspace, 16)))
-    return fail(ATF_ERR_WORKSPACE, "workspace of %zu bytes (16-byte aligned) required, got %zu", need,
-                workspace ? workspace_bytes : 0);
-  a.ws_ml = static_cast<float*>(workspace);
-  a.ws_o = need > 0 ? a.ws_ml + static_cast<size_t>(batch) * num_kv_heads * a.n_splits * atf::kDecMaxGroup * 2
-                    : nullptr;
+  if (int r = set_workspace(workspace, workspace_bytes, &a)) return r;
   hipError_t e = atf::launch_decode(a, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "decode launch");
   return ok();
@@ -346,6 +363,36 @@ int atf_decode_paged_slices_bf16(void* out, int64_t o_sb, int64_t o_sh, const vo
   return decode_with_workspace(out, o_sb, o_sh, q, q_sb, q_sh, kv_cache, num_pages, page_table, max_pages,
                                seq_lens, batch, num_q_heads, num_kv_heads, max_seq_len, zhi_slice, true, sm_scale,
                                rope_cs, rope_max_pos, layout, workspace, workspace_bytes, stream);
+}
+
+int atf_decode_rows_bf16(void* out, int64_t o_sb, int64_t o_sh, const void* q, int64_t q_sb, int64_t q_sh,
+                         const void* k, int64_t ks_b, int64_t ks_t, int64_t ks_h, const void* v, int64_t vs_b,
+                         int64_t vs_t, int64_t vs_h, int batch, int num_q_heads, int num_kv_heads, int seq_len,
+                         const int32_t* zhi, int zhi_entries, float sm_scale, const float* rope_cs, int rope_max_pos,
+                         int layout, void* workspace, size_t workspace_bytes, void* stream) {
+  if (batch < 0) return fail(ATF_ERR_INVALID, "batch must be >= 0");
+  if (batch == 0) return ok();
+  if (!out || !q || !k || !v) return fail(ATF_ERR_INVALID, "null pointer argument");
+  if (int r = check_decode_heads(num_q_heads, num_kv_heads, seq_len)) return r;
+  if (zhi && zhi_entries != ATF_LEVELS && zhi_entries != ATF_SLICES)
+    return fail(ATF_ERR_INVALID, "window table must have %d or %d entries, got %d", ATF_LEVELS, ATF_SLICES, zhi_entries);
+  if (!aligned(k, 16) || !aligned(v, 16)) return fail(ATF_ERR_INVALID, "k and v must be 16-byte aligned");
+  for (int64_t s : {ks_b, ks_t, ks_h, vs_b, vs_t, vs_h})
+    if (s % 8 != 0) return fail(ATF_ERR_INVALID, "source strides must be multiples of 8 elements");
+  // a block's 16 rows are addressed with 31-bit byte offsets
+  for (int64_t s : {ks_t, vs_t})
+    if (s < 0 || s > (int64_t(1) << 26))
+      return fail(ATF_ERR_UNSUPPORTED, "token strides of k and v must be between 0 and 2^26 elements");
+  atf::DecodeArgs a{};
+  if (int r = decode_prepare_query(out, o_sb, o_sh, q, q_sb, q_sh, batch, num_q_heads, num_kv_heads, seq_len, zhi,
+                                   zhi_entries == ATF_SLICES, sm_scale, rope_cs, rope_max_pos, layout, &a))
+    return r;
+  if (int r = set_workspace(workspace, workspace_bytes, &a)) return r;
+  const atf::DecodeRows rows{static_cast<const uint16_t*>(k), static_cast<const uint16_t*>(v), ks_b, ks_t, ks_h,
+                             vs_b, vs_t, vs_h};
+  hipError_t e = atf::launch_decode_rows(a, rows, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return hip_fail(e, "decode launch");
+  return ok();
 }
 
 int atf_decode_paged_bf16_noalloc(void* out, int64_t o_sb, int64_t o_sh, const void* q, int64_t q_sb, int64_t q_sh,

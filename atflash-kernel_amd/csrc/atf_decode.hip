@@ -191,6 +191,47 @@ __device__ __forceinline__ void dec_load_page(const DecHot& a, int h, int raw, b
   dec_load_v(a, ref, lane, r.v);
 }
 
+// A split's wave partials (m, l, o), in LDS, combined by log-sum-exp: the output
+// where the split is the whole sequence, otherwise the split's partial for
+// decode_merge_kernel.  Thread t owns query heads t / 32 + 2 kWaves j, dims
+// 4 (t % 32) .. +3.
+template <int kWaves>
+__device__ __forceinline__ void store_split(const DecodeArgs& a, int s, int h, int b, int hkv, const float* sh_o,
+                                            const float* sh_m, const float* sh_l) {
+  const float NEG_INF = -__builtin_huge_valf();
+  const float c = a.scale_log2;
+  const int tid = threadIdx.x;
+  const int d4 = 4 * (tid & 31);
+  const int64_t pbase = (static_cast<int64_t>(b) * hkv + h) * a.n_splits * kDecMaxGroup;  // split 0, head 0
+  for (int gq = tid >> 5; gq < a.group; gq += 2 * kWaves) {
+    float M = NEG_INF;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) M = fmaxf(M, sh_m[w * kDecMaxGroup + gq]);
+    float L = 0.f;
+    f32x4 acc = f32x4{};
+    if (M != NEG_INF) {
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) {
+        const float wt = fast_exp2((sh_m[w * kDecMaxGroup + gq] - M) * c);  // empty wave: m = -inf -> 0
+        L += wt * sh_l[w * kDecMaxGroup + gq];
+        acc += wt * *reinterpret_cast<const f32x4*>(&sh_o[(w * kDecMaxGroup + gq) * kD + d4]);
+      }
+    }
+    if (a.n_splits == 1) {  // the split is the whole sequence: write the output
+      const float inv = L > 0.f ? 1.f / L : 0.f;
+      uint16_t* out = a.out + static_cast<int64_t>(b) * a.o_sb + static_cast<int64_t>(h * a.group + gq) * a.o_sh + d4;
+      u32x2 pk;
+      pk[0] = pack_bf16x2(acc[0] * inv, acc[1] * inv);
+      pk[1] = pack_bf16x2(acc[2] * inv, acc[3] * inv);
+      *reinterpret_cast<u32x2*>(out) = pk;
+    } else {  // the split's partial, merged by decode_merge_kernel
+      const int64_t pi = pbase + static_cast<int64_t>(s) * kDecMaxGroup + gq;
+      *reinterpret_cast<f32x4*>(a.ws_o + pi * kD + d4) = acc;
+      if (d4 == 0) *reinterpret_cast<f32x2*>(a.ws_ml + pi * 2) = f32x2{M, L};
+    }
+  }
+}
+
 // two waves per SIMD: at most 256 registers per wave.  kWaves = 8 (one
 // workgroup per CU) or 4 (short contexts: smaller splits over more CUs).
 template <bool kPerKey, int kWaves>
@@ -394,36 +435,238 @@ void decode_kernel(const int32_t* page_table, const int32_t* seq_lens, const uin
     }
   }
   __syncthreads();
-  // thread t owns query heads t / 32 + 2 kWaves j, dims 4 (t % 32) .. +3
-  const int d4 = 4 * (tid & 31);
-  const int64_t pbase = (static_cast<int64_t>(b) * hot.hkv + h) * a.n_splits * kDecMaxGroup;  // split 0, head 0
-  for (int gq = tid >> 5; gq < a.group; gq += 2 * kWaves) {
-    float M = NEG_INF;
+  store_split<kWaves>(a, s, h, b, hot.hkv, sh_o, sh_m, sh_l);
+}
+
+// ---- decode over contiguous K and V rows ----
+// The same decode reading a sequence's K and V as rows [token][128] with strides,
+// as the reference's decode call passes them, instead of a paged cache: K
+// (rotated here when rope_cs is given) and V are read once, where packing them
+// into pages first reads them, writes them and reads them again.  Blocks of 16
+// tokens take the place of pages, and everything else (window rules, splits,
+// waves, MFMA operands, merge) is decode_kernel's, so the outputs are those of
+// the packed cache bit for bit.
+//   K: lane (token t = lane % 16, g = lane / 16) reads slices g, 4 + g, 8 + g and
+// 12 + g of its token's row: 16 bytes each (sorted-pair rows), or 8 + 8 (the two
+// halves of the slice's pairs in half-split rows).  A slice past the page's
+// window, or of a token past the sequence, is read at an offset past the buffer
+// range: zeros, no request.
+//   V: lane (g, i = lane % 16) reads dims 8i..8i+7 of tokens 4g..4g+3 (16 lanes
+// read whole 256-byte rows); MFMA e takes element e of each, four tokens deep,
+// so its row i is dim 8i + e and the transposition is two byte permutes per MFMA.
+//   HBM bound.  Against the call that packs first (28 / 4 heads, k = 2, pre-rotated
+// rows): 32K tokens 71.2 -> 18.6 us (26.5 us of writer, 18.5 us of decode and
+// merge, and the host's allocations and copies before); 128K OFF 50.9 us a call.
+struct RowsArgs {
+  DecodeArgs d;  // page fields unused; d.max_seq_len is the length of every sequence
+  DecodeRows r;
+};
+
+constexpr uint32_t kRowsRange = 0x7fffffffu;  // buffer range of a block's rows
+constexpr uint32_t kRowsSkip = 0x80000000u;   // an offset past it
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(const void* base) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, static_cast<int>(kRowsRange), kBufferWord3);
+}
+
+template <bool kRope>
+struct RowBlock {
+  u32x4 k[4];
+  u32x4 v[4];
+  u32x4 cs[kRope ? 8 : 1];  // (cos, sin) of the four slices' pairs
+};
+
+// kHalf: half-split rows (kRope implies it), otherwise sorted-pair rows.
+// kU: blocks in flight per wave (with RoPE two: their (cos, sin) take as many
+// registers as K and V).
+template <bool kPerKey, bool kHalf, bool kRope, int kWaves>
+__global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2)))
+void decode_rows_kernel(RowsArgs ra) {
+  constexpr int kU = kRope ? 2 : 4;
+  static_assert(kDecUnroll % kU == 0 && (kHalf || !kRope), "rows kernel");
+  const DecodeArgs& a = ra.d;
+  __shared__ __attribute__((aligned(16))) float sh_o[kWaves * kDecMaxGroup * kD];
+  __shared__ float sh_m[kWaves * kDecMaxGroup], sh_l[kWaves * kDecMaxGroup];
+  const int s = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int g = lane >> 4, t = lane & 15;
+  const int N = a.max_seq_len;
+  PageOrder ord = page_order(s, a.n_splits, a.pages_per_split);
+  set_page_count(ord, s, a.n_splits, a.pages_per_split, (N + kPage - 1) / kPage);
+  const float NEG_INF = -__builtin_huge_valf();
+  const float c = a.scale_log2;
+  // the wave's blocks in decode_kernel's order: block j of the wave is local
+  // page kDecUnroll (w + kWaves (j / kDecUnroll)) + j % kDecUnroll of the split
+  auto local = [&](int j) { return kDecUnroll * (wave + kWaves * (j / kDecUnroll)) + j % kDecUnroll; };
+
+  const uint8_t* kbase = reinterpret_cast<const uint8_t*>(ra.r.k + b * ra.r.ks_b + h * ra.r.ks_h);
+  const uint8_t* vbase = reinterpret_cast<const uint8_t*>(ra.r.v + b * ra.r.vs_b + h * ra.r.vs_h);
+  const int64_t kt = 2 * ra.r.ks_t, vt = 2 * ra.r.vs_t;  // bytes per token
+  uint32_t koff[4];
+  int zl[4];  // distance limits of the lane's slices (page rule: level 0 has none)
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) M = fmaxf(M, sh_m[w * kDecMaxGroup + gq]);
-    float L = 0.f;
-    f32x4 acc = f32x4{};
-    if (M != NEG_INF) {
+  for (int lp = 0; lp < 4; ++lp) {
+    const int sl = 4 * lp + g;
+    koff[lp] = static_cast<uint32_t>(t * kt) + 2 * (kHalf ? slice_pair0(sl) : 8 * sl);
+    zl[lp] = 0;
 #pragma unroll
-      for (int w = 0; w < kWaves; ++w) {
-        const float wt = fast_exp2((sh_m[w * kDecMaxGroup + gq] - M) * c);  // empty wave: m = -inf -> 0
-        L += wt * sh_l[w * kDecMaxGroup + gq];
-        acc += wt * *reinterpret_cast<const f32x4*>(&sh_o[(w * kDecMaxGroup + gq) * kD + d4]);
+    for (int i = 0; i < 4; ++i)
+      if (g == i) zl[lp] = (!kPerKey && 4 * lp + i < 2) ? INT32_MAX : a.st.zhi[4 * lp + i];
+  }
+
+  auto load_k = [&](int p, RowBlock<kRope>& r) {
+    const int n0 = p * kPage;
+    const int z = max(0, (N - 1) - (n0 + kPage - 1));  // the youngest key's age
+    const auto rk = rows_rsrc(kbase + n0 * kt);
+    const bool in = n0 + t < N;
+#pragma unroll
+    for (int lp = 0; lp < 4; ++lp) {
+      const bool on = in && zl[lp] >= z;
+      if constexpr (kHalf) {
+        const u32x2 x1 = __builtin_bit_cast(
+            u32x2, __builtin_amdgcn_raw_buffer_load_b64(rk, on ? koff[lp] : kRowsSkip, 0, kLoadStream));
+        const u32x2 x2 = __builtin_bit_cast(
+            u32x2, __builtin_amdgcn_raw_buffer_load_b64(rk, on ? koff[lp] + 2 * kP : kRowsSkip, 0, kLoadStream));
+        r.k[lp] = u32x4{x1[0], x1[1], x2[0], x2[1]};
+      } else {
+        r.k[lp] = __builtin_bit_cast(
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, on ? koff[lp] : kRowsSkip, 0, kLoadStream));
       }
     }
-    if (a.n_splits == 1) {  // the split is the whole sequence: write the output
-      const float inv = L > 0.f ? 1.f / L : 0.f;
-      uint16_t* out = a.out + static_cast<int64_t>(b) * a.o_sb + static_cast<int64_t>(h * a.group + gq) * a.o_sh + d4;
-      u32x2 pk;
-      pk[0] = pack_bf16x2(acc[0] * inv, acc[1] * inv);
-      pk[1] = pack_bf16x2(acc[2] * inv, acc[3] * inv);
-      *reinterpret_cast<u32x2*>(out) = pk;
-    } else {  // the split's partial, merged by decode_merge_kernel
-      const int64_t pi = pbase + static_cast<int64_t>(s) * kDecMaxGroup + gq;
-      *reinterpret_cast<f32x4*>(a.ws_o + pi * kD + d4) = acc;
-      if (d4 == 0) *reinterpret_cast<f32x2*>(a.ws_ml + pi * 2) = f32x2{M, L};
+    if constexpr (kRope) {
+      const auto rc = rows_rsrc(a.rope_cs + static_cast<int64_t>(n0) * (2 * kP));
+#pragma unroll
+      for (int lp = 0; lp < 4; ++lp) {
+        const bool on = in && zl[lp] >= z;
+        const uint32_t off = t * (kP * 8) + slice_pair0(4 * lp + g) * 8;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          r.cs[2 * lp + i] = __builtin_bit_cast(
+              u32x4, __builtin_amdgcn_raw_buffer_load_b128(rc, on ? off + 16 * i : kRowsSkip, 0, 0));
+      }
+    }
+  };
+  auto load_v = [&](int p, RowBlock<kRope>& r) {
+    const int n0 = p * kPage;
+    const auto rv = rows_rsrc(vbase + n0 * vt);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t off = static_cast<uint32_t>((4 * g + i) * vt) + 16 * t;
+      r.v[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                             rv, n0 + 4 * g + i < N ? off : kRowsSkip, 0, kLoadStream));
+    }
+  };
+  RowBlock<kRope> blk[kU];
+#pragma unroll
+  for (int u = 0; u < kU; ++u)
+    if (local(u) < ord.count) {
+      const int p = ord.po + ord.pm * local(u);
+      load_k(p, blk[u]);
+      load_v(p, blk[u]);
+    }
+
+  // Q as decode_kernel loads it
+  u32x4 Qf[4];
+  {
+    const int qh = h * a.group + min(t, a.group - 1);
+    const uint16_t* qrow = a.q + b * a.q_sb + qh * a.q_sh;
+    load_slices4<4>(qrow, kHalf ? kLayoutHalfSplit : kLayoutSortedPair, g, Qf);
+    if constexpr (kRope) {
+#pragma unroll
+      for (int lp = 0; lp < 4; ++lp) {
+        float cs[8];
+        load_cs4(a.rope_cs, N - 1, slice_pair0(4 * lp + g), cs);
+        Qf[lp] = rope_slice(Qf[lp], cs);
+      }
+    }
+#pragma unroll
+    for (int lp = 0; lp < 4; ++lp)
+      if (t >= a.group) Qf[lp] = u32x4{0u, 0u, 0u, 0u};
+  }
+
+  f32x4 O[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) O[e] = f32x4{};
+  float m_run = NEG_INF, l_run = 0.f;
+  for (int j0 = 0; local(j0) < ord.count; j0 += kU) {
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      if (local(j0 + u) >= ord.count) break;
+      RowBlock<kRope>& r = blk[u];
+      const int n0 = (ord.po + ord.pm * local(j0 + u)) * kPage;
+      // slices past the window: of the key (per-key rule) or of the page's youngest key
+      const int age = kPerKey ? (N - 1) - (n0 + t) : max(0, (N - 1) - (n0 + kPage - 1));
+      f32x4 S = f32x4{};
+#pragma unroll
+      for (int lp = 0; lp < 4; ++lp) {
+        u32x4 K = r.k[lp];
+        if constexpr (kRope) {
+          float cs[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) cs[i] = __uint_as_float(r.cs[2 * lp + (i >> 2)][i & 3]);
+          K = rope_slice(K, cs);
+        }
+        if (age > zl[lp]) K = u32x4{0u, 0u, 0u, 0u};
+        S = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, K), __builtin_bit_cast(bf16x8, Qf[lp]), S, 0,
+                                                    0, 0);
+      }
+      const int jn = local(j0 + kU + u);
+      const bool reload = jn < ord.count;
+      if (reload) load_k(ord.po + ord.pm * jn, r);
+      // S: query head lane % 16, tokens 4 (lane / 16) + i
+      float mx = NEG_INF;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (n0 + 4 * g + i >= N) S[i] = NEG_INF;
+        mx = fmaxf(mx, S[i]);
+      }
+      mx = quad_max(mx);
+      const bool grow = (mx - m_run) * c > 8.f;  // the lazy reference max of decode_kernel
+      if (__builtin_amdgcn_ballot_w64(grow) != 0) {
+        const float alpha = !grow ? 1.f : (m_run == NEG_INF ? 0.f : fast_exp2((m_run - mx) * c));
+        l_run *= alpha;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) O[e] *= alpha;
+        m_run = grow ? mx : m_run;
+      }
+      const float msc = (m_run == NEG_INF) ? 0.f : m_run * c;
+      float pv[4];
+      float ls = 0.f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        pv[i] = fast_exp2(__builtin_fmaf(S[i], c, -msc));
+        ls += pv[i];
+      }
+      l_run += ls;
+      const s16x4 pb = __builtin_bit_cast(s16x4, u32x2{pack_bf16x2(pv[0], pv[1]), pack_bf16x2(pv[2], pv[3])});
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const uint32_t sel = (e & 1) ? 0x07060302u : 0x05040100u;  // the odd or even halves of two words
+        const u32x2 col = {__builtin_amdgcn_perm(r.v[1][e >> 1], r.v[0][e >> 1], sel),
+                           __builtin_amdgcn_perm(r.v[3][e >> 1], r.v[2][e >> 1], sel)};
+        O[e] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, col), pb, O[e], 0, 0, 0);
+      }
+      if (reload) load_v(ord.po + ord.pm * jn, r);
     }
   }
+
+  const float l_tot = quad_sum(l_run);
+  if (t < a.group) {
+    // O[e][i]: dim 8 (4g + i) + e
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float* o = &sh_o[(wave * kDecMaxGroup + t) * kD + 8 * (4 * g + i)];
+      *reinterpret_cast<f32x4*>(o) = f32x4{O[0][i], O[1][i], O[2][i], O[3][i]};
+      *reinterpret_cast<f32x4*>(o + 4) = f32x4{O[4][i], O[5][i], O[6][i], O[7][i]};
+    }
+    if (lane < 16) {
+      sh_m[wave * kDecMaxGroup + t] = m_run;
+      sh_l[wave * kDecMaxGroup + t] = l_tot;
+    }
+  }
+  __syncthreads();
+  store_split<kWaves>(a, s, h, b, a.hkv, sh_o, sh_m, sh_l);
 }
 
 // ---- measurement probe: the streaming ceiling of the decode's page loads ----
@@ -675,6 +918,15 @@ __global__ void decode_page_levels_kernel(int32_t* out, int n_pages, int N, Leve
   out[p] = levels_of(lt, max(0, (N - 1) - (p * kPage + kPage - 1)));
 }
 
+// The merge of a call's split partials (nothing to do with one split).
+static hipError_t launch_merge(const DecodeArgs& a, hipStream_t s) {
+  if (a.n_splits == 1) return hipSuccess;
+  hipLaunchKernelGGL(decode_merge_kernel, dim3(kMergeChunks, a.hkv, a.batch), dim3(512), 0, s,
+                     static_cast<const float*>(a.ws_ml), static_cast<const float*>(a.ws_o), a.out, a.o_sb, a.o_sh,
+                     a.n_splits, a.group, a.hkv, a.scale_log2);
+  return hipGetLastError();
+}
+
 hipError_t launch_decode(const DecodeArgs& a, hipStream_t s) {
   if (a.batch <= 0) return hipSuccess;
   const dim3 grid(a.n_splits, a.hkv, a.batch);
@@ -687,12 +939,31 @@ hipError_t launch_decode(const DecodeArgs& a, hipStream_t s) {
     if (a.per_key) ATF_DEC_LAUNCH(true, 4); else ATF_DEC_LAUNCH(false, 4);
   }
 #undef ATF_DEC_LAUNCH
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || a.n_splits == 1) return e;
-  hipLaunchKernelGGL(decode_merge_kernel, dim3(kMergeChunks, a.hkv, a.batch), dim3(512), 0, s,
-                     static_cast<const float*>(a.ws_ml), static_cast<const float*>(a.ws_o), a.out, a.o_sb, a.o_sh,
-                     a.n_splits, a.group, a.hkv, a.scale_log2);
-  return hipGetLastError();
+  if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+  return launch_merge(a, s);
+}
+
+hipError_t launch_decode_rows(const DecodeArgs& a, const DecodeRows& r, hipStream_t s) {
+  if (a.batch <= 0) return hipSuccess;
+  const dim3 grid(a.n_splits, a.hkv, a.batch);
+  const RowsArgs ra{a, r};
+#define ATF_ROWS_LAUNCH(PK, HALF, ROPE)                                                                  \
+  do {                                                                                                   \
+    if (a.waves == 8)                                                                                    \
+      hipLaunchKernelGGL((decode_rows_kernel<PK, HALF, ROPE, 8>), grid, dim3(512), 0, s, ra);            \
+    else                                                                                                 \
+      hipLaunchKernelGGL((decode_rows_kernel<PK, HALF, ROPE, 4>), grid, dim3(256), 0, s, ra);            \
+  } while (0)
+  if (a.rope_cs != nullptr) {
+    if (a.per_key) ATF_ROWS_LAUNCH(true, true, true); else ATF_ROWS_LAUNCH(false, true, true);
+  } else if (a.layout == kLayoutHalfSplit) {
+    if (a.per_key) ATF_ROWS_LAUNCH(true, true, false); else ATF_ROWS_LAUNCH(false, true, false);
+  } else {
+    if (a.per_key) ATF_ROWS_LAUNCH(true, false, false); else ATF_ROWS_LAUNCH(false, false, false);
+  }
+#undef ATF_ROWS_LAUNCH
+  if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+  return launch_merge(a, s);
 }
 
 // ---- fixed scratch for the entry point that allocates nothing ----

@@ -86,6 +86,13 @@ struct DecodeArgs {
   float* ws_o;         // [B][Hkv][n_splits][16][128]
 };
 
+// K and V of a contiguous decode: rows [batch][token][head][128] (element strides).
+struct DecodeRows {
+  const uint16_t* k;
+  const uint16_t* v;
+  int64_t ks_b, ks_t, ks_h, vs_b, vs_t, vs_h;
+};
+
 hipError_t launch_kv_write(const KvWriteArgs& a, hipStream_t s);
 hipError_t launch_prefill(const PrefillArgs& a, hipStream_t s);
 // The MFMA-ceiling probe of the prefill (measurement only): sink holds
@@ -94,6 +101,8 @@ hipError_t launch_prefill_mfma_probe(float* sink, int nq, int hq, hipStream_t s)
 hipError_t launch_prefill_tile_levels(int32_t* out, int n_row_tiles, int n_kblocks, int q_offset,
                                       const LevelTable& lt, hipStream_t s);
 hipError_t launch_decode(const DecodeArgs& a, hipStream_t s);
+// The decode over contiguous rows; every sequence has a.max_seq_len tokens.
+hipError_t launch_decode_rows(const DecodeArgs& a, const DecodeRows& r, hipStream_t s);
 // launch_decode with the workspace pointers taken from the device's fixed
 // scratch (a.ws_ml and a.ws_o are set here).
 hipError_t launch_decode_noalloc(DecodeArgs a, hipStream_t s);

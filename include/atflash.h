@@ -174,6 +174,27 @@ int atf_decode_paged_slices_bf16(void* out, int64_t o_sb, int64_t o_sh,
                                  void* stream);
 
 /*
+ * The same decode over contiguous K and V, read in place: k and v are bf16
+ * [batch][seq_len][num_kv_heads][128] with element strides (token, head and
+ * batch strides multiples of 8; 16-byte aligned; last dim contiguous; token
+ * strides at most 2^26, else ATF_ERR_UNSUPPORTED), every sequence of seq_len
+ * tokens, the query at position seq_len - 1.  rope_cs, when given, rotates q and
+ * k (half-split rows).  zhi: the level table (zhi_entries = ATF_LEVELS, per
+ * 16-token block) or the per-slice table (ATF_SLICES, per key); NULL means window
+ * OFF.  Workspace as atf_decode_workspace_bytes(batch, ..., seq_len).
+ *
+ * Replaces single_decode_with_kv_cache_with_jit_module on the contiguous cache
+ * the reference passes (kernels/flashinfer_port/fiwin_common.py:96-112,
+ * e2e_pipeline/atflash_e2e_fafi.py:106-109).
+ */
+int atf_decode_rows_bf16(void* out, int64_t o_sb, int64_t o_sh, const void* q, int64_t q_sb, int64_t q_sh,
+                         const void* k, int64_t ks_b, int64_t ks_t, int64_t ks_h,
+                         const void* v, int64_t vs_b, int64_t vs_t, int64_t vs_h,
+                         int batch, int num_q_heads, int num_kv_heads, int seq_len,
+                         const int32_t* zhi, int zhi_entries, float sm_scale, const float* rope_cs,
+                         int rope_max_pos, int layout, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * atf_decode_paged_bf16 for callers that cannot allocate device memory (code
  * under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  It has no counterpart in the reference.  Same arguments and
