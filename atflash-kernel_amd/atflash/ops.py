@@ -145,7 +145,7 @@ def _decode_workspace(device, handle, B, hq, hkv, max_seq_len, L):
     if nbytes is None:
         if len(_WS_BYTES) >= 4096:
             _WS_BYTES.clear()
-        nbytes = _WS_BYTES[shape] = int(L.atf_decode_workspace_bytes(B, hq, hkv, max_seq_len))
+        nbytes = _WS_BYTES[shape] = int(L.atf_decode_workspace_bytes_even(B, hq, hkv, max_seq_len))
     key = (device.index, handle)
     ws = _DECODE_WS.get(key)
     if ws is None or ws[1] < nbytes:
@@ -288,7 +288,7 @@ class DecodePlan:
         self.device = kv_cache.device
         self.shape = (B, Hq, D)
         self.q_strides = (q_sb, q_sh, 1)
-        nbytes = int(L.atf_decode_workspace_bytes(B, Hq, kv_cache.shape[1], int(max_seq_len)))
+        nbytes = int(L.atf_decode_workspace_bytes_even(B, Hq, kv_cache.shape[1], int(max_seq_len)))
         self._ws = torch.empty((max(nbytes, 16) + 3) // 4, dtype=torch.float32, device=self.device)
         self._keep = (kv_cache, page_table, seq_lens, rope_cs)  # the tensors the addresses point into
         self._table = _lib.zhi_array(None if zhi is None else tuple(zhi), _lib.SLICES if slices else _lib.LEVELS)

@@ -2,6 +2,7 @@
 // kernel launches.  Declarations and documentation: include/atflash.h.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -128,6 +129,29 @@ size_t partial_bytes(int batch, int hkv, int ns) {
   return static_cast<size_t>(batch) * hkv * ns * atf::kDecMaxGroup * (atf::kD + 2) * sizeof(float);
 }
 
+// Runs per kv head of a batch split evenly (decode_batch_kernel), 0 where the
+// splits of decode_split are used.  The lengths are not known here; a batch of
+// equal lengths that decode_split fits to the chip gains nothing by the runs and
+// pays two extra round trips and a few more partials (2 us a call: 6% of 8 x 8K
+// tokens at 8 kv heads, 2.6% of 16 x 8K, 0.3% of 8 x 32K), where a ragged one
+// gains 1.1 to 2 times.  So, by the batch's pages if every sequence were as long
+// as the longest: from 96K pages (768 MB of K and V) on; from 48K on where
+// decode_split's workgroups overfill the chip (12 x 8K tokens: 288 workgroups
+// over 256 CUs, 77 us against 63; 40 x 8K: 320, 215 against 182).  Not for one
+// sequence, nor from 512 sequence x kv head pairs on (two workgroups a CU and no
+// merge: 64 x 8K at 8 kv heads 276 us against 291).
+int batch_runs(int batch, int hkv, int max_seq_len) {
+  const int64_t pairs = static_cast<int64_t>(batch) * hkv;
+  const int64_t pages = pairs * ((static_cast<int64_t>(max_seq_len) + atf::kPage - 1) / atf::kPage);
+  if (batch <= 1 || pairs >= 512) return 0;
+  const bool overfull = (256 + pairs - 1) / pairs * pairs * 20 > 256 * 21;  // 5% past 256 workgroups
+  if (pages < (overfull ? 48 : 96) * 1024) return 0;
+  return std::max(1, atf::kDecBatchWgs / hkv);
+}
+size_t batch_bytes(int hkv, int runs) {
+  return static_cast<size_t>(hkv) * runs * 2 * atf::kDecMaxGroup * (atf::kD + 2) * sizeof(float);
+}
+
 }  // namespace
 
 extern "C" {
@@ -234,6 +258,13 @@ size_t atf_decode_workspace_bytes(int batch, int num_q_heads, int num_kv_heads, 
   return partial_bytes(batch, num_kv_heads, ns);
 }
 
+size_t atf_decode_workspace_bytes_even(int batch, int num_q_heads, int num_kv_heads, int max_seq_len) {
+  const size_t need = atf_decode_workspace_bytes(batch, num_q_heads, num_kv_heads, max_seq_len);
+  if (batch <= 0 || num_kv_heads <= 0 || max_seq_len <= 0) return need;
+  const int runs = batch_runs(batch, num_kv_heads, max_seq_len);
+  return runs == 0 ? need : std::max(need, batch_bytes(num_kv_heads, runs));
+}
+
 }  // extern "C"
 
 namespace {
@@ -305,6 +336,16 @@ int decode_prepare(void* out, int64_t o_sb, int64_t o_sh, const void* q, int64_t
                               slice_table, sm_scale, rope_cs, rope_max_pos, layout, a);
 }
 
+// The paged decode's workspace: a batch is split evenly if it holds that split's partials.
+int set_batch_workspace(void* workspace, size_t workspace_bytes, atf::DecodeArgs* a) {
+  const int runs = batch_runs(a->batch, a->hkv, a->max_seq_len);
+  if (runs == 0 || !workspace || !aligned(workspace, 16) || workspace_bytes < batch_bytes(a->hkv, runs)) return 0;
+  a->runs = runs;
+  a->ws_ml = static_cast<float*>(workspace);
+  a->ws_o = a->ws_ml + static_cast<size_t>(a->hkv) * runs * 2 * atf::kDecMaxGroup * 2;
+  return runs;
+}
+
 // The caller's workspace -> the split partials' addresses.
 int set_workspace(void* workspace, size_t workspace_bytes, atf::DecodeArgs* a) {
   const size_t need = partial_bytes(a->batch, a->hkv, a->n_splits);
@@ -334,7 +375,8 @@ int decode_with_workspace(void* out, int64_t o_sb, int64_t o_sh, const void* q, 
                              seq_lens, batch, num_q_heads, num_kv_heads, max_seq_len, zhi, slice_table, sm_scale,
                              rope_cs, rope_max_pos, layout, &a))
     return r;
-  if (int r = set_workspace(workspace, workspace_bytes, &a)) return r;
+  if (!set_batch_workspace(workspace, workspace_bytes, &a))
+    if (int r = set_workspace(workspace, workspace_bytes, &a)) return r;
   hipError_t e = atf::launch_decode(a, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "decode launch");
   return ok();

@@ -195,14 +195,14 @@ __device__ __forceinline__ void dec_load_page(const DecHot& a, int h, int raw, b
 // where the split is the whole sequence, otherwise the split's partial for
 // decode_merge_kernel.  Thread t owns query heads t / 32 + 2 kWaves j, dims
 // 4 (t % 32) .. +3.
+// part: the partial's index in the workspace; whole: the split is the sequence.
 template <int kWaves>
-__device__ __forceinline__ void store_split(const DecodeArgs& a, int s, int h, int b, int hkv, const float* sh_o,
-                                            const float* sh_m, const float* sh_l) {
+__device__ __forceinline__ void store_split(const DecodeArgs& a, int64_t part, bool whole, int h, int b,
+                                            const float* sh_o, const float* sh_m, const float* sh_l) {
   const float NEG_INF = -__builtin_huge_valf();
   const float c = a.scale_log2;
   const int tid = threadIdx.x;
   const int d4 = 4 * (tid & 31);
-  const int64_t pbase = (static_cast<int64_t>(b) * hkv + h) * a.n_splits * kDecMaxGroup;  // split 0, head 0
   for (int gq = tid >> 5; gq < a.group; gq += 2 * kWaves) {
     float M = NEG_INF;
 #pragma unroll
@@ -217,7 +217,7 @@ __device__ __forceinline__ void store_split(const DecodeArgs& a, int s, int h, i
         acc += wt * *reinterpret_cast<const f32x4*>(&sh_o[(w * kDecMaxGroup + gq) * kD + d4]);
       }
     }
-    if (a.n_splits == 1) {  // the split is the whole sequence: write the output
+    if (whole) {  // write the output
       const float inv = L > 0.f ? 1.f / L : 0.f;
       uint16_t* out = a.out + static_cast<int64_t>(b) * a.o_sb + static_cast<int64_t>(h * a.group + gq) * a.o_sh + d4;
       u32x2 pk;
@@ -225,46 +225,23 @@ __device__ __forceinline__ void store_split(const DecodeArgs& a, int s, int h, i
       pk[1] = pack_bf16x2(acc[2] * inv, acc[3] * inv);
       *reinterpret_cast<u32x2*>(out) = pk;
     } else {  // the split's partial, merged by decode_merge_kernel
-      const int64_t pi = pbase + static_cast<int64_t>(s) * kDecMaxGroup + gq;
+      const int64_t pi = part * kDecMaxGroup + gq;
       *reinterpret_cast<f32x4*>(a.ws_o + pi * kD + d4) = acc;
       if (d4 == 0) *reinterpret_cast<f32x2*>(a.ws_ml + pi * 2) = f32x2{M, L};
     }
   }
 }
 
-// two waves per SIMD: at most 256 registers per wave.  kWaves = 8 (one
-// workgroup per CU) or 4 (short contexts: smaller splits over more CUs).
+// Decode of one split (pages `ord`) of sequence b: this wave's pages, its partial
+// (m, l, o) into LDS.  ent: the page-table entries of the wave's first group;
+// wave: its index in the workgroup.
 template <bool kPerKey, int kWaves>
-__global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2)))
-void decode_kernel(const int32_t* page_table, const int32_t* seq_lens, const uint16_t* kv_cache, int max_pages,
-                   int pages_per_split, int max_seq_len, int hkv, int num_pages, int n_splits, DecodeArgs a) {
-  const DecHot hot{page_table, seq_lens, kv_cache, max_pages, pages_per_split, max_seq_len, hkv, num_pages, n_splits};
-  // wave partials
-  __shared__ __attribute__((aligned(16))) float sh_o[kWaves * kDecMaxGroup * kD];
-  __shared__ float sh_m[kWaves * kDecMaxGroup], sh_l[kWaves * kDecMaxGroup];
-
-  const int s = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-  const int tid = threadIdx.x;
-  const int wave = tid >> 6, lane = tid & 63;
-  const int g = lane & 15;
-  // Local page indices: wave w takes the groups of kDecUnroll local pages that
-  // start at kDecUnroll * (w + kWaves * i); local page j is page po + pm * j.
+__device__ __forceinline__ void decode_pages(const DecHot& hot, const DecodeArgs& a, int h, int b, int N,
+                                             const int32_t* row, const PageOrder& ord, int wave, int p_first,
+                                             int (&ent)[kDecUnroll], float* sh_o, float* sh_m, float* sh_l) {
   constexpr int kStride = kDecUnroll * kWaves;
-  const int p_first = kDecUnroll * __builtin_amdgcn_readfirstlane(wave);
-  PageOrder ord = page_order(s, hot.n_splits, hot.pages_per_split);
-  const int po = ord.po, pm = ord.pm;
-  // The first group's page-table entries are fetched together with the
-  // sequence length, their index clamped into the table row only (an entry
-  // past the split is never used), so the first page loads wait for two
-  // memory round trips after the kernel arguments, not three.
-  int ent[kDecUnroll];
-  const int32_t* row = hot.page_table + static_cast<int64_t>(b) * hot.max_pages;
-#pragma unroll
-  for (int u = 0; u < kDecUnroll; ++u) ent[u] = row[min(po + pm * (p_first + u), hot.max_pages - 1)];
-  const int N = max(0, min(hot.seq_lens[b], hot.max_seq_len));
-  const int n_pages = (N + kPage - 1) / kPage;
-  set_page_count(ord, s, hot.n_splits, hot.pages_per_split, n_pages);
-  const int p_end = ord.count;
+  const int p_end = ord.count, po = ord.po, pm = ord.pm;
+  const int lane = threadIdx.x & 63, g = lane & 15;
   const float NEG_INF = -__builtin_huge_valf();
   const float c = a.scale_log2;
 
@@ -434,8 +411,203 @@ void decode_kernel(const int32_t* page_table, const int32_t* seq_lens, const uin
       sh_l[wave * kDecMaxGroup + g] = l_tot;
     }
   }
+}
+
+// two waves per SIMD: at most 256 registers per wave.  kWaves = 8 (one
+// workgroup per CU) or 4 (short contexts: smaller splits over more CUs).
+template <bool kPerKey, int kWaves>
+__global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2)))
+void decode_kernel(const int32_t* page_table, const int32_t* seq_lens, const uint16_t* kv_cache, int max_pages,
+                   int pages_per_split, int max_seq_len, int hkv, int num_pages, int n_splits, DecodeArgs a) {
+  const DecHot hot{page_table, seq_lens, kv_cache, max_pages, pages_per_split, max_seq_len, hkv, num_pages, n_splits};
+  // wave partials
+  __shared__ __attribute__((aligned(16))) float sh_o[kWaves * kDecMaxGroup * kD];
+  __shared__ float sh_m[kWaves * kDecMaxGroup], sh_l[kWaves * kDecMaxGroup];
+
+  const int s = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
+  const int tid = threadIdx.x;
+  const int wave = tid >> 6;
+  // Local page indices: wave w takes the groups of kDecUnroll local pages that
+  // start at kDecUnroll * (w + kWaves * i); local page j is page po + pm * j.
+  const int p_first = kDecUnroll * __builtin_amdgcn_readfirstlane(wave);
+  PageOrder ord = page_order(s, hot.n_splits, hot.pages_per_split);
+  const int po = ord.po, pm = ord.pm;
+  // The first group's page-table entries are fetched together with the
+  // sequence length, their index clamped into the table row only (an entry
+  // past the split is never used), so the first page loads wait for two
+  // memory round trips after the kernel arguments, not three.
+  int ent[kDecUnroll];
+  const int32_t* row = hot.page_table + static_cast<int64_t>(b) * hot.max_pages;
+#pragma unroll
+  for (int u = 0; u < kDecUnroll; ++u) ent[u] = row[min(po + pm * (p_first + u), hot.max_pages - 1)];
+  const int N = max(0, min(hot.seq_lens[b], hot.max_seq_len));
+  const int n_pages = (N + kPage - 1) / kPage;
+  set_page_count(ord, s, hot.n_splits, hot.pages_per_split, n_pages);
+  decode_pages<kPerKey, kWaves>(hot, a, h, b, N, row, ord, wave, p_first, ent, sh_o, sh_m, sh_l);
   __syncthreads();
-  store_split<kWaves>(a, s, h, b, hot.hkv, sh_o, sh_m, sh_l);
+  store_split<kWaves>(a, (static_cast<int64_t>(b) * hot.hkv + h) * a.n_splits + s, a.n_splits == 1, h, b, sh_o, sh_m, sh_l);
+}
+
+// ---- a batch split evenly over the chip ----
+// decode_kernel's grid gives every sequence of a batch the splits of the longest
+// one, as many as fit 256 workgroups: a ragged batch leaves most workgroups with
+// little to do, and sequence x kv head counts that do not divide 256 either leave
+// CUs idle or start a second wave of workgroups (12 sequences x 8 kv heads: 288).
+// Here the pages of the whole batch, one sequence after the other, are cut into
+// `chunks` equal runs per kv head (kDecBatchWgs = 256 workgroups in all, one per
+// CU), and workgroup (c, h) decodes run c: the end of one sequence, whole ones,
+// the beginning of another.  The lengths live in device memory, so every
+// workgroup derives its run from them (one load per 64 sequences, sums by DPP).
+// A sequence inside one run is written by its workgroup; a cut one leaves a
+// partial per run, merged by decode_merge_kernel<true>.  Run c's partials are 2c
+// (of a sequence that it begins with) and 2c + 1 (of one that begins inside it).
+//   HBM bound.  Measured against decode_kernel on the same batch (24 / 8 heads,
+// vec8 k = 2; us a call): 12 sequences of 700 to 32768 tokens 110 -> 73, 16 of
+// them 157 -> 80, 12 of 32K 266 -> 202, 40 of 8K 214 -> 185, 8 of 32K (equal, 256
+// splits either way) 134.6 -> 135.8.  512 workgroups of 4 waves instead: ragged
+// batches the same within 6%, equal ones of 32K 5% slower.
+struct BatchPlan {
+  int run;   // virtual pages per run
+  int gran;  // a sequence takes a multiple of this many virtual pages
+  int nsb;   // > 0: nearly equal lengths; every sequence takes nsb runs, interleaved page by page
+};
+
+// Lengths of the 64 sequences from b0 on, one per lane (0 past the batch).
+__device__ __forceinline__ int batch_lens(const int32_t* seq_lens, int batch, int max_seq_len, int b0) {
+  const int b = b0 + static_cast<int>(threadIdx.x & 63);
+  return b < batch ? max(0, min(seq_lens[b], max_seq_len)) : 0;
+}
+__device__ __forceinline__ int len_pages(int n) { return (n + kPage - 1) / kPage; }
+
+// Inclusive prefix sum (or maximum) over the wave's 64 lanes by DPP (VALU moves:
+// row shifts by 1, 2, 4, 8, then the row broadcasts); lane 63 has the total.
+template <class Op>
+__device__ __forceinline__ int wave_scan(int x, const Op& op) {
+  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, true));
+  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, true));
+  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, true));
+  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, true));
+  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false));
+  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false));
+  return x;
+}
+__device__ __forceinline__ int scan_sum(int x) {
+  return wave_scan(x, [](int a, int b) { return a + b; });
+}
+
+// The runs of a batch; every wave computes the same plan.  lens0: batch_lens of
+// the first 64 sequences.
+//   Short batches (each sequence's pages by the 32 fit the runs): runs of 32
+// pages, one 4-page group per wave, no run across two sequences.
+//   Nearly equal lengths (the longest within 4% of the mean) that divide the
+// runs (5% left over at most): each sequence in nsb splits of its own,
+// interleaved page by page as decode_kernel's are.
+//   Otherwise equal runs, in groups of 4 pages.
+__device__ __forceinline__ BatchPlan batch_plan(const int32_t* seq_lens, int batch, int max_seq_len, int chunks,
+                                                int lens0) {
+  constexpr int kRun = kDecUnroll * kDecBatchWaves;  // one 4-page group per wave
+  int t4 = 0, tr = 0, mx = 0;
+  for (int b0 = 0; b0 < batch; b0 += 64) {
+    const int p = len_pages(b0 == 0 ? lens0 : batch_lens(seq_lens, batch, max_seq_len, b0));
+    t4 += __builtin_amdgcn_readlane(scan_sum((p + 3) & ~3), 63);
+    tr += __builtin_amdgcn_readlane(scan_sum((p + kRun - 1) / kRun), 63);
+    mx = max(mx, __builtin_amdgcn_readlane(wave_scan(p, [](int a, int b) { return max(a, b); }), 63));
+  }
+  if (tr <= chunks) return BatchPlan{kRun, kRun, 0};
+  const int nsb = chunks / batch;
+  if (nsb > 0 && static_cast<int64_t>(mx) * batch * 100 <= static_cast<int64_t>(t4) * 104 &&
+      nsb * batch * 20 >= chunks * 19)
+    return BatchPlan{0, 0, nsb};
+  return BatchPlan{((t4 + chunks - 1) / chunks + 3) & ~3, 4, 0};
+}
+
+// The first sequence that ends past virtual page `at` (find) or sequence `at`,
+// the virtual page x it starts at, and its 64 sequences' lengths (lens; lens0 on
+// entry).  b = batch if there is none.
+__device__ __forceinline__ void batch_locate(const int32_t* seq_lens, int batch, int max_seq_len, int gran, bool find,
+                                             int at, int& lens, int& b, int& x) {
+  const int lane = threadIdx.x & 63;
+  int base = 0;
+  for (int b0 = 0; b0 < batch; b0 += 64) {
+    if (b0 > 0) lens = batch_lens(seq_lens, batch, max_seq_len, b0);
+    const int v = (len_pages(lens) + gran - 1) & ~(gran - 1);
+    const int incl = scan_sum(v);
+    const uint64_t hit = __builtin_amdgcn_ballot_w64(find ? base + incl > at : b0 + lane == at);
+    if (hit != 0) {
+      const int l = __builtin_ctzll(hit);
+      b = b0 + l;
+      x = base + __builtin_amdgcn_readlane(incl - v, l);
+      return;
+    }
+    base += __builtin_amdgcn_readlane(incl, 63);
+  }
+  b = batch;
+  x = base;
+}
+
+template <bool kPerKey>
+__global__ __launch_bounds__(kDecBatchWaves * 64) __attribute__((amdgpu_waves_per_eu(2)))
+void decode_batch_kernel(const int32_t* page_table, const int32_t* seq_lens, const uint16_t* kv_cache, int max_pages,
+                         int chunks, int max_seq_len, int hkv, int num_pages, int batch, DecodeArgs a) {
+  constexpr int kWaves = kDecBatchWaves;
+  const DecHot hot{page_table, seq_lens, kv_cache, max_pages, 0, max_seq_len, hkv, num_pages, 1};
+  __shared__ __attribute__((aligned(16))) float sh_o[kWaves * kDecMaxGroup * kD];
+  __shared__ float sh_m[kWaves * kDecMaxGroup], sh_l[kWaves * kDecMaxGroup];
+  const int c = blockIdx.x + gridDim.x * blockIdx.z, h = blockIdx.y;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int p_first = kDecUnroll * wave;
+  int lens = batch_lens(seq_lens, batch, max_seq_len, 0);
+  // The first group's page-table entries if the lengths turn out nearly equal
+  // (this run: split s of sequence bu, interleaved), fetched with the lengths,
+  // their index clamped into the table row: that case then waits for no more
+  // memory round trips than decode_kernel does.
+  const int nsb = chunks / batch;
+  const int bu = nsb > 0 ? min(c / nsb, batch - 1) : 0, su = nsb > 0 ? c - c / nsb * nsb : 0;
+  int ent[kDecUnroll];
+#pragma unroll
+  for (int u = 0; u < kDecUnroll; ++u)
+    ent[u] = page_table[static_cast<int64_t>(bu) * max_pages + min(su + max(nsb, 1) * (p_first + u), max_pages - 1)];
+  const BatchPlan bp = batch_plan(seq_lens, batch, max_seq_len, chunks, lens);
+  int b, x = 0;
+  const int begin = c * bp.run, end = begin + bp.run;
+  if (bp.nsb > 0) {
+    b = c / bp.nsb;
+    if (b >= 64) lens = batch_lens(seq_lens, batch, max_seq_len, b & ~63);
+  } else {
+    batch_locate(seq_lens, batch, max_seq_len, bp.gran, true, begin, lens, b, x);
+  }
+  bool first = true;
+  while (b < batch && (bp.nsb > 0 ? first : x < end)) {
+    const int N = __builtin_amdgcn_readlane(lens, b & 63);
+    const int P = len_pages(N);
+    PageOrder ord;
+    bool whole;
+    if (bp.nsb > 0) {
+      const int s = c - b * bp.nsb;
+      ord = PageOrder{s, bp.nsb, P > s ? (P - s + bp.nsb - 1) / bp.nsb : 0};
+      whole = bp.nsb == 1;
+    } else {
+      const int p0 = max(begin - x, 0), p1 = min(end - x, P);
+      ord = PageOrder{p0, 1, max(p1 - p0, 0)};
+      whole = p0 == 0 && p1 == P;
+    }
+    if (ord.count > 0 || bp.nsb > 0) {
+      if (!first) __syncthreads();  // the last sequence's partials in LDS have been read
+      const int32_t* row = page_table + static_cast<int64_t>(b) * max_pages;
+      if (bp.nsb == 0) {
+#pragma unroll
+        for (int u = 0; u < kDecUnroll; ++u) ent[u] = dec_fetch_entry(row, ord, p_first + u);
+      }
+      decode_pages<kPerKey, kWaves>(hot, a, h, b, N, row, ord, wave, p_first, ent, sh_o, sh_m, sh_l);
+      __syncthreads();
+      const int64_t part = static_cast<int64_t>(h) * 2 * chunks + 2 * c + (bp.nsb == 0 && x > begin ? 1 : 0);
+      store_split<kWaves>(a, part, whole, h, b, sh_o, sh_m, sh_l);
+      first = false;
+    }
+    if (bp.nsb > 0) break;
+    x += (P + bp.gran - 1) & ~(bp.gran - 1);
+    if ((++b & 63) == 0) lens = batch_lens(seq_lens, batch, max_seq_len, b);
+  }
 }
 
 // ---- decode over contiguous K and V rows ----
@@ -666,7 +838,7 @@ void decode_rows_kernel(RowsArgs ra) {
     }
   }
   __syncthreads();
-  store_split<kWaves>(a, s, h, b, a.hkv, sh_o, sh_m, sh_l);
+  store_split<kWaves>(a, (static_cast<int64_t>(b) * a.hkv + h) * a.n_splits + s, a.n_splits == 1, h, b, sh_o, sh_m, sh_l);
 }
 
 // ---- measurement probe: the streaming ceiling of the decode's page loads ----
@@ -846,38 +1018,69 @@ __device__ __forceinline__ void merge_lane_groups(float& m, float& l, f32x4& o, 
   }
 }
 
+// kBatch: the partials of decode_batch_kernel (n_splits holds the runs per kv
+// head); a sequence in one run has its output already, an empty one is zeroed here.
+template <bool kBatch>
 __global__ __launch_bounds__(512) void decode_merge_kernel(const float* ws_ml, const float* ws_o, uint16_t* out,
                                                             int64_t o_sb, int64_t o_sh, int n_splits, int group,
-                                                            int hkv, float scale_log2) {
-  const MergeArgs a{ws_ml, ws_o, out, o_sb, o_sh, n_splits, group, hkv, scale_log2};
+                                                            int hkv, float scale_log2, const int32_t* seq_lens,
+                                                            int batch, int max_seq_len) {
+  MergeArgs a{ws_ml, ws_o, out, o_sb, o_sh, n_splits, group, hkv, scale_log2};
   const int chunk = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
+  int64_t part0 = (static_cast<int64_t>(b) * a.hkv + h) * a.n_splits;  // split 0's partial
+  int step = 1, skew = 0;  // split i's is part0 + step * i, less skew after the first
   const int tid = threadIdx.x;
   const float NEG_INF = -__builtin_huge_valf();
   const float c = a.scale_log2;
-  const int64_t pbase = (static_cast<int64_t>(b) * a.hkv + h) * a.n_splits * kDecMaxGroup;  // split 0, head 0
   const int H = (a.group <= 8) ? kMergeRowsPerWave : kMergeRowsPerWave / 2;
   const int row = tid / kMergeLanes;  // (head, split group)
   const int mg = row / H, hh = row - (row / H) * H;
   const int q4 = 4 * (tid % kMergeLanes);
   const int md4 = chunk * kMergeDims + q4;
   const bool mact = mg < a.group;
+  f32x2 mlv[kMergeBatch];
+  f32x4 ov[kMergeBatch];
+  auto load = [&](int j0) {
+#pragma unroll
+    for (int j = 0; j < kMergeBatch; ++j) {
+      const int sp = j0 + j * H;
+      mlv[j] = f32x2{NEG_INF, 0.f};
+      ov[j] = f32x4{};
+      if (mact && sp < a.n_splits) {
+        const int64_t pi = (part0 + step * sp - (sp > 0 ? skew : 0)) * kDecMaxGroup + mg;
+        mlv[j] = *reinterpret_cast<const f32x2*>(a.ws_ml + pi * 2);
+        ov[j] = *reinterpret_cast<const f32x4*>(a.ws_o + pi * kD + md4);
+      }
+    }
+  };
+  if constexpr (kBatch) {
+    // The partials of the nearly-equal-lengths layout are loaded along with the
+    // lengths that decide whether it is the one (if not, they are not used).
+    int lens = batch_lens(seq_lens, batch, max_seq_len, 0);
+    const int nsb = n_splits / batch;
+    part0 = static_cast<int64_t>(h) * 2 * n_splits + 2 * b * nsb;
+    step = 2;
+    a.n_splits = nsb;
+    load(hh);
+    const BatchPlan bp = batch_plan(seq_lens, batch, max_seq_len, n_splits, lens);
+    if (bp.nsb == 0) {
+      int bb = b, x = 0;
+      batch_locate(seq_lens, batch, max_seq_len, bp.gran, false, b, lens, bb, x);
+      const int c0 = x / bp.run, P = len_pages(__builtin_amdgcn_readlane(lens, b & 63));
+      a.n_splits = P > 0 ? (x + P - 1) / bp.run - c0 + 1 : 0;
+      skew = x > c0 * bp.run ? 1 : 0;
+      part0 = static_cast<int64_t>(h) * 2 * n_splits + 2 * c0 + skew;
+    }
+    if (a.n_splits == 1) return;
+    if (bp.nsb == 0) load(hh);
+  } else {
+    load(hh);
+  }
   float m_t = NEG_INF, L_t = 0.f;
   f32x4 acc_t = f32x4{};
   if (mact) {
     for (int j0 = hh; j0 < a.n_splits; j0 += kMergeBatch * H) {
-      f32x2 mlv[kMergeBatch];
-      f32x4 ov[kMergeBatch];
-#pragma unroll
-      for (int j = 0; j < kMergeBatch; ++j) {
-        const int sp = j0 + j * H;
-        mlv[j] = f32x2{NEG_INF, 0.f};
-        ov[j] = f32x4{};
-        if (sp < a.n_splits) {
-          const int64_t pi = pbase + static_cast<int64_t>(sp) * kDecMaxGroup + mg;
-          mlv[j] = *reinterpret_cast<const f32x2*>(a.ws_ml + pi * 2);
-          ov[j] = *reinterpret_cast<const f32x4*>(a.ws_o + pi * kD + md4);
-        }
-      }
+      if (j0 != hh) load(j0);
       float mb = m_t;
 #pragma unroll
       for (int j = 0; j < kMergeBatch; ++j) mb = fmaxf(mb, mlv[j][0]);
@@ -920,15 +1123,37 @@ __global__ void decode_page_levels_kernel(int32_t* out, int n_pages, int N, Leve
 
 // The merge of a call's split partials (nothing to do with one split).
 static hipError_t launch_merge(const DecodeArgs& a, hipStream_t s) {
-  if (a.n_splits == 1) return hipSuccess;
-  hipLaunchKernelGGL(decode_merge_kernel, dim3(kMergeChunks, a.hkv, a.batch), dim3(512), 0, s,
-                     static_cast<const float*>(a.ws_ml), static_cast<const float*>(a.ws_o), a.out, a.o_sb, a.o_sh,
-                     a.n_splits, a.group, a.hkv, a.scale_log2);
+  const dim3 grid(kMergeChunks, a.hkv, a.batch);
+#define ATF_MERGE_LAUNCH(BATCH, N)                                                                                 \
+  hipLaunchKernelGGL(decode_merge_kernel<BATCH>, grid, dim3(512), 0, s, static_cast<const float*>(a.ws_ml),       \
+                     static_cast<const float*>(a.ws_o), a.out, a.o_sb, a.o_sh, N, a.group, a.hkv, a.scale_log2,   \
+                     a.seq_lens, a.batch, a.max_seq_len)
+  if (a.runs > 0) ATF_MERGE_LAUNCH(true, a.runs);
+  else if (a.n_splits > 1) ATF_MERGE_LAUNCH(false, a.n_splits);
+  else return hipSuccess;
+#undef ATF_MERGE_LAUNCH
   return hipGetLastError();
 }
 
 hipError_t launch_decode(const DecodeArgs& a, hipStream_t s) {
   if (a.batch <= 0) return hipSuccess;
+  if (a.runs > 0) {
+    // Block order: the runs of a sequence, then the kv heads, then the sequences,
+    // as decode_kernel's, where equal lengths give a sequence four runs or more
+    // (16 sequences of 32K, 4 kv heads: 138 us; all runs of a head side by side:
+    // 145) and no run is left over (its empty workgroups would upset the even
+    // spread over the CUs: 5 sequences of 32K, 8 kv heads: 130 us against 115);
+    // otherwise the latter (64 of 8K, 4 kv heads: 149 against 157).
+    const int nsb = a.runs / a.batch, side = nsb >= 4 && nsb * a.batch == a.runs ? nsb : a.runs;
+    const dim3 grid(side, a.hkv, a.runs / side);
+#define ATF_BATCH_LAUNCH(PK)                                                                                        \
+  hipLaunchKernelGGL(decode_batch_kernel<PK>, grid, dim3(kDecBatchWaves * 64), 0, s, a.page_table, a.seq_lens,     \
+                     a.kv_cache, a.max_pages, a.runs, a.max_seq_len, a.hkv, a.num_pages, a.batch, a)
+    if (a.per_key) ATF_BATCH_LAUNCH(true); else ATF_BATCH_LAUNCH(false);
+#undef ATF_BATCH_LAUNCH
+    if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    return launch_merge(a, s);
+  }
   const dim3 grid(a.n_splits, a.hkv, a.batch);
 #define ATF_DEC_LAUNCH(PK, W)                                                                                   \
   hipLaunchKernelGGL((decode_kernel<PK, W>), grid, dim3(W * 64), 0, s, a.page_table, a.seq_lens, a.kv_cache,    \
