@@ -33,7 +33,11 @@ COMMON = [
 # that the dispatch preloads into SGPRs (kernarg preloading, gfx950): up to 14
 # dwords (16 user SGPRs less the argument-block pointer).  A firmware without
 # it runs the compiler's compatibility prologue, which loads them instead.
-EXTRA = {"atf_decode.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=14"]}
+# The prefill's one-wave-per-SIMD kernel may use all 512 registers of a SIMD
+# lane; its MFMAs keep their results in ordinary registers (left to itself the
+# compiler puts them in accumulation registers there and copies every score out).
+EXTRA = {"atf_decode.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=14"],
+         "atf_prefill.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
 def sources():

@@ -4,7 +4,8 @@
 // _flash_attn_fwd(q, k, v, causal=True, atflash_window_zhi=zhi),
 // microbench/b1_correctness.py:84-85, e2e_pipeline/atflash_e2e_fafi.py:118-119).
 //
-// Work decomposition
+// Work decomposition (prefill_kernel; prefill_solo_kernel below takes launches
+// that would leave CUs idle)
 //   workgroup = 8 waves = 256 consecutive query positions of one q head;
 //   wave      = 32 positions (one MFMA row block).  Waves w and w+4 share a SIMD
 //               and run one phase apart ("ping-pong"): at every step one of them
@@ -177,6 +178,39 @@ __device__ __forceinline__ void lds_copy_page(const uint8_t* base, uint32_t nbyt
                "buffer_load_dwordx4 %1, %2, 0 offen offset:3072 lds\n\t"
                "s_mov_b32 m0, %0"
                : "=&s"(saved) : "v"(voff), "s"(rs), "s"(la) : "memory");
+}
+
+// lds_copy_page row by row: the resource and LDS address once per page, then row
+// kRow (1 KB) wherever the caller has room for it.
+struct PageCopy {
+  u32x4 rs;
+  uint32_t la;
+};
+__device__ __forceinline__ PageCopy page_copy(const uint8_t* base, uint32_t nbytes, lds_u8* dst) {
+  const uint64_t ad = reinterpret_cast<uint64_t>(base);
+  PageCopy p;
+  p.la = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(dst)));
+  p.rs[0] = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(ad)));
+  p.rs[1] = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(ad >> 32))) & 0xffffu;
+  p.rs[2] = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(nbytes));
+  p.rs[3] = static_cast<uint32_t>(kBufferWord3);
+  return p;
+}
+template <int kRow>
+__device__ __forceinline__ void copy_row(const PageCopy& p, uint32_t voff) {
+  uint32_t saved;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\t"
+               "buffer_load_dwordx4 %1, %2, 0 offen offset:%4 lds\n\t"
+               "s_mov_b32 m0, %0"
+               : "=&s"(saved) : "v"(voff), "s"(p.rs), "s"(p.la), "n"(kRow * 1024) : "memory");
+}
+__device__ __forceinline__ void copy_row_n(const PageCopy& p, uint32_t voff, int r) {
+  switch (r) {
+    case 0: copy_row<0>(p, voff); break;
+    case 1: copy_row<1>(p, voff); break;
+    case 2: copy_row<2>(p, voff); break;
+    default: copy_row<3>(p, voff); break;
+  }
 }
 
 __device__ __forceinline__ void zero_page(lds_u8* dst, int lane) {
@@ -769,6 +803,384 @@ __global__ __launch_bounds__(kPfWaves * 64, 1) void prefill_kernel(PrefillArgs a
   }
 }
 
+// ---- one wave per SIMD: launches that leave CUs idle ----
+
+// PV of the previous tile pair (P in Pf, V at vb) with the softmax of the
+// current one (scores in S) between its MFMAs, P replaced in place page by
+// page as its PV steps have read it.  Reads the first QK operands ahead.
+template <bool kRaw, class Copy>
+__device__ __forceinline__ float pv_softmax_stream(const lds_u8* vb, const lds_u8* kb, bf16x8 (&Pf)[8], f32x16 (&O)[4],
+                                                   const f32x16 (&S)[4], float c, bf16x8 (&f)[kRing], const Copy& copy) {
+  constexpr int kLag = 3;  // step k's P goes to page k/4, last read by MFMA 4 (k/4) + 3
+  float lt = 0.f, p0 = 0.f, p1 = 0.f;
+  auto pack = [&](int k) {
+    u32x4 w = __builtin_bit_cast(u32x4, Pf[k >> 2]);
+    w[k & 3] = pack_bf16x2(p0, p1);
+    Pf[k >> 2] = __builtin_bit_cast(bf16x8, w);
+    lt += p0 + p1;
+    asm volatile("" : "+v"(lt));  // the sum stays here: sunk below the stream, its 64 terms would stay live
+  };
+  auto exps = [&](int k) {
+    const f32x16& Sk = S[k >> 3];
+    const int e = 2 * (k & 7);
+    p0 = fast_exp2(kRaw ? Sk[e] * c : Sk[e]);
+    p1 = fast_exp2(kRaw ? Sk[e + 1] * c : Sk[e + 1]);
+  };
+  exps(0);
+#pragma unroll
+  for (int i = 0; i < 32; ++i) {
+    f[(i + kRing - 1) % kRing] = lds_frag(stream_src(vb, kb, i + kRing - 1));
+    __builtin_amdgcn_sched_barrier(0);
+    O[i & 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[i % kRing], Pf[i >> 2], O[i & 3], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    copy(i);
+    if (i >= kLag) {
+      pack(i - kLag);
+      __builtin_amdgcn_sched_barrier(0);
+      exps(i - kLag + 1);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+#pragma unroll
+  for (int k = 32 - kLag; k < 32; ++k) {
+    pack(k);
+    if (k < 31) exps(k + 1);
+  }
+  return lt;
+}
+
+// qk_stream with copy(r), r = 0..7, spread over it.
+template <int L, class Copy>
+__device__ __forceinline__ void qk_stream_copy(const lds_u8* kb, bf16x8 (&f)[kRing], const u32x4 (&Qf)[kLevels],
+                                               const f32x16& C, f32x16 (&S)[4], const Copy& copy) {
+  constexpr int NS = 32 + 4 * L;
+#pragma unroll
+  for (int i = 32; i < NS; ++i) {
+    if (i + kRing - 1 < NS) f[(i + kRing - 1) % kRing] = lds_frag(stream_src(kb, kb, i + kRing - 1));
+    __builtin_amdgcn_sched_barrier(0);
+    const int j = i - 32;
+    S[j & 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[i % kRing], __builtin_bit_cast(bf16x8, Qf[j >> 2]),
+                                                       (j >> 2) == 0 ? C : S[j & 3], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+      if (j == r * 4 * L / 8) copy(r);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// S of the four 32-key blocks of a pair with a level count of its own each
+// (byte j of lm): one chain per block, a runtime loop over its levels.
+__device__ __forceinline__ void qk_blocks(uint64_t lm, const lds_u8* kb, const u32x4 (&Qf)[kLevels], const f32x16& C,
+                                          f32x16 (&S)[4]) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const uint32_t m = (static_cast<uint32_t>(lm >> (8 * j)) & 0xffu) | 1u;  // levels as bits 0..L-1 (table order)
+    S[j] = C;
+#pragma unroll
+    for (int l = 0; l < kLevels; ++l)
+      if ((m >> l) & 1u)
+        S[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lds_frag(kb + j * 8192 + l * 512),
+                                                       __builtin_bit_cast(bf16x8, Qf[l]), S[j], 0, 0, 0);
+  }
+}
+
+// The same attention with 128 query rows per workgroup: 4 waves of 32 rows, one
+// per SIMD, for launches whose 128-row workgroups all fit the chip at once
+// (prefill_solo).  prefill_kernel's 256-row workgroups would leave half of the
+// CUs idle or more there.  Without a partner on its SIMD, a wave overlaps its own
+// work: the softmax of pair u sits between the MFMAs of the PV of pair u-1, which
+// it does not depend on (pv_softmax_stream), then come the rescale check and the
+// QK of pair u+1; one barrier per pair.  The copies are spread over the MFMAs row
+// by row, V of pair u during its PV part, K of pair u+3 during its QK part, and
+// the scalar work (level counts, page addresses) is done between them.  Every
+// sum and every rescale is formed in prefill_kernel's order, so both give the
+// same bits, and chunked prefill those of a single shot.
+//   What bounds it: the LDS operand reads (4 waves x 1 KB per 32-cycle MFMA are
+// the LDS' 128 bytes a clock) and, in the PV part, one wave's issue of 32 MFMAs,
+// 64 exps, 64 adds and 32 packings (about 60 cycles an MFMA).  1024 queries behind
+// 32K keys, 28 / 4 heads: k = 2 531 -> 431 us, OFF 602 -> 472; 517 tokens 29 -> 20; where the chip is
+// full it loses (4096 tokens 127 -> 152 us), a pair taking 3100 to 3500 cycles for
+// 32 rows of a SIMD where prefill_kernel takes 5000 to 5700 for 64.
+constexpr int kSoloWaves = 4;
+constexpr int kSoloRowsWg = kSoloWaves * kPfRowsWave;
+template <bool kRaw>
+__global__ __launch_bounds__(kSoloWaves * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
+void prefill_solo_kernel(PrefillArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem_raw[];
+  lds_u8* smem = (lds_u8*)(smem_raw);
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int b, h, qt;
+  if (!prefill_block(a, blockIdx.x, b, h, qt)) return;
+  const int kvh = h / a.group;
+
+  const int lr0_wg = qt * kSoloRowsWg;
+  const int lr0 = lr0_wg + wave * kPfRowsWave;
+  const int pos0_wg = a.q_offset + lr0_wg;
+  const int pos0 = a.q_offset + lr0;
+  const int n_ktiles = (a.nk + kPfTileN - 1) / kPfTileN;
+  const int last_wg = a.q_offset + min(a.nq, lr0_wg + kSoloRowsWg) - 1;
+  const int T = min(n_ktiles, last_wg / kPfTileN + 1);
+  const int U = (T + 1) >> 1;
+  const int t_end =
+      (lr0 < a.nq) ? min(n_ktiles, (a.q_offset + min(a.nq, lr0 + kPfRowsWave) - 1) / kPfTileN + 1) : 0;
+
+  // page-table entries of 64 pages (8 tile pairs) at a time, one per lane
+  const int n_pages_k = (a.nk + kPage - 1) / kPage;
+  const int32_t* prow = a.page_table + static_cast<int64_t>(b) * a.max_pages;
+  auto fetch64 = [&](int chunk) {
+    const int p = chunk * 64 + lane;
+    int v = prow[min(p, n_pages_k - 1)];
+    return (p < n_pages_k && v >= 0 && v < a.num_pages) ? v : -1;
+  };
+  int tab_k = fetch64(0);
+  int tab_n = fetch64(1);
+  int tab_v = tab_k;
+
+  u32x4 Qf[kLevels];
+  const bool second = lane >= 32;
+  const int row = lr0 + (lane & 31);
+  {
+    const int row_c = min(row, a.nq - 1);
+    const uint16_t* qrow = a.q + static_cast<int64_t>(b) * a.q_sb + static_cast<int64_t>(row_c) * a.q_st +
+                           static_cast<int64_t>(h) * a.q_sh;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      u32x4 v[4];
+      const int s0 = 8 * j + (second ? 1 : 0);
+      load_slices4<2>(qrow, a.layout, s0, v);
+      if (a.rope_cs != nullptr) {
+        float cs[4][8];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) load_cs4(a.rope_cs, a.q_offset + row_c, slice_pair0(s0 + 2 * i), cs[i]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = rope_slice(v[i], cs[i], a.scale_log2);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) Qf[4 * j + i] = (row < a.nq) ? v[i] : u32x4{0u, 0u, 0u, 0u};
+    }
+  }
+
+  f32x16 O[4];
+#pragma unroll
+  for (int db = 0; db < 4; ++db) O[db] = f32x16{};
+  const float NEG_INF = -__builtin_huge_valf();
+  float m_ref = 0.f, l_run = 0.f;
+  f32x16 Cm = f32x16{};
+  const float c = a.scale_log2;
+  const float inv_c = 1.f / c;
+
+  // Level counts.  Level i of a 32-key block m (keys 32m..32m+31) is read from
+  // m = ceil((pos0 - 31 - zhi[i]) / 32) on (LevelWalker's rule in 32-key units).
+  // Lane 8j + i holds that block less an offset, so that one compare and ballot
+  // per iteration (against 4u + 4) counts the levels of the four blocks of pair
+  // u + 1 (bytes 0..3 of the mask) and of the nearer blocks of the two tiles of
+  // pair u + 3 for the workgroup's first row (bytes 4, 5: the rows to stage).
+  int tl;
+  {
+    int z = 0;
+#pragma unroll
+    for (int i = 0; i < kLevels; ++i) z = (lane & 7) == i ? min(a.lt.zhi[i], 1 << 30) : z;
+    const int j = lane >> 3;
+    const int first = ((j < 4 ? pos0 : pos0_wg) - z) >> 5;  // ceil((pos0 - 31 - z) / 32)
+    tl = j < 4 ? first - j : (j == 4 ? first - 9 : (j == 5 ? first - 11 : INT32_MAX));
+  }
+  auto level_mask = [&](int u) { return __builtin_amdgcn_ballot_w64(tl <= 4 * u + 4); };
+  auto count = [](uint64_t m, int j) {  // D_eff >= 16: at least one level
+    const int n = __builtin_popcount(static_cast<uint32_t>(m >> (8 * j)) & 0xffu);
+    return n < 1 ? 1 : n;
+  };
+
+  const uint32_t k_off = static_cast<uint32_t>(k_copy_src(lane)), v_off = static_cast<uint32_t>(v_copy_src(lane));
+  const int k_lane = ((lane & 31) >> 4) * 4096 + (lane >> 5) * 256 + (lane & 15) * 16;
+  const int v_lane = (lane >> 5) * 512 + (lane & 31) * 16;
+  const uint8_t* vbase = reinterpret_cast<const uint8_t*>(a.kv_cache) + static_cast<size_t>(kvh) * (kKvBlockElems * 2);
+  const uint8_t* kbase = vbase + kKHalfElems * 2;
+  const uint32_t pstride = static_cast<uint32_t>(a.hkv) * (kKvBlockElems * 2u);
+
+  // Copy of half hh of pair p (tile 2p + hh, this wave's page): always four row
+  // loads; a missing page or a pair past the end has an empty range (zeros).
+  auto k_page = [&](int p, int hh, int rows) {
+    const int pg = __builtin_amdgcn_readlane(tab_k, (8 * p + 4 * hh + wave) & 63);
+    return page_copy(kbase + static_cast<size_t>(static_cast<uint32_t>(pg < 0 ? 0 : pg)) * pstride,
+                     pg < 0 || p >= U ? 0u : static_cast<uint32_t>(rows) * 1024u,
+                     smem + (p % kPfKPairs) * kPfPairBytes + hh * kPfSlotBytes + wave * 4096);
+  };
+  auto v_page = [&](int p, int hh) {
+    const int pg = __builtin_amdgcn_readlane(tab_v, (8 * p + 4 * hh + wave) & 63);
+    return page_copy(vbase + static_cast<size_t>(static_cast<uint32_t>(pg < 0 ? 0 : pg)) * pstride, pg < 0 || p >= U ? 0u : 4096u,
+                     smem + kPfVRegion + (p & 1) * kPfPairBytes + hh * kPfSlotBytes + wave * 4096);
+  };
+
+  // ---- prologue: K of pairs 0..2; QK of pair 0 ----
+#pragma unroll
+  for (int p = 0; p < 3; ++p) {
+    const uint64_t lm = level_mask(p - 3);
+    const PageCopy c0 = k_page(p, 0, (count(lm, 4) + 1) >> 1), c1 = k_page(p, 1, (count(lm, 5) + 1) >> 1);
+#pragma unroll
+    for (int r = 0; r < 8; ++r) copy_row_n(r < 4 ? c0 : c1, k_off, r & 3);
+  }
+  // V pair 1: read by the first PV with P = 0
+  zero_page(smem + kPfVRegion + kPfPairBytes + wave * 4096, lane);
+  zero_page(smem + kPfVRegion + kPfPairBytes + kPfSlotBytes + wave * 4096, lane);
+  __builtin_amdgcn_s_waitcnt(kWaitVm | 8);  // K of pairs 0 and 1
+  pf_barrier();
+  f32x16 S[4];
+  uint64_t lm = level_mask(-1);
+  {
+    const lds_u8* kb = smem + k_lane;
+    qk_blocks(lm, kb, Qf, Cm, S);
+  }
+  bf16x8 Pf[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) Pf[i] = bf16x8{};
+  // The wave's copies: its V pages of pair u (prepared an iteration ahead) and its
+  // K pages of pair u + 3.
+  PageCopy va = v_page(0, 0), vb2 = v_page(0, 1), ka, kb2;
+  for (int u = 0; u < U; ++u) {
+    const int kp = u + 3;
+    if ((kp & 7) == 0) {
+      tab_k = tab_n;
+      tab_n = fetch64((kp >> 3) + 1);
+    }
+    auto hook_pv = [&](int i) {
+      if (i < 8) copy_row_n(i < 4 ? va : vb2, v_off, i & 3);
+      if (i == 12) lm = level_mask(u);
+      if (i == 16) ka = k_page(kp, 0, (count(lm, 4) + 1) >> 1);
+      if (i == 20) kb2 = k_page(kp, 1, (count(lm, 5) + 1) >> 1);
+    };
+    auto hook_qk = [&](int r) {
+      copy_row_n(r < 4 ? ka : kb2, k_off, r & 3);
+      if (r == 7) {
+        if (((u + 1) & 7) == 0) tab_v = tab_k;
+        va = v_page(u + 1, 0);
+        vb2 = v_page(u + 1, 1);
+      }
+    };
+    const lds_u8* kb = smem + ((u + 1) % kPfKPairs) * kPfPairBytes + k_lane;
+    const lds_u8* vb = smem + kPfVRegion + ((u + 1) & 1) * kPfPairBytes + v_lane;
+    if (__builtin_expect((2 * u + 2) * kPfTileN - 1 > pos0 || (2 * u + 2) * kPfTileN > a.nk, 0)) {
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh) {
+        const int n0 = (2 * u + hh) * kPfTileN;
+        // element (kb, r) holds key n0 + 4*(lane/32) + 32kb + 8(r/4) + r%4; masked
+        // when key > min(row position, nk - 1), every key of a tile past t_end
+        const int thr = 2 * u + hh >= t_end ? -1 : min(pos0 + (lane & 31), a.nk - 1) - n0 - 4 * (lane >> 5);
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            S[2 * hh + kk][r] = (32 * kk + 8 * (r >> 2) + (r & 3) > thr) ? NEG_INF : S[2 * hh + kk][r];
+      }
+    }
+    bf16x8 f[kRing];
+    pv_prefetch(vb, f);
+    float lt = pv_softmax_stream<kRaw>(vb, kb, Pf, O, S, c, f, hook_pv);
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64((u == 0) || !(lt <= 256.f)) != 0, 0)) {
+      float mx = NEG_INF;
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, S[kk][r]);
+      mx = pair_max(mx);
+      if (kRaw) mx *= c;
+      // (a wave past the queries has no key to set its reference max by)
+      const bool grow = (u == 0 && t_end > 0) || mx > kLazyRescaleLog2;
+      if (__builtin_amdgcn_ballot_w64(grow) != 0) {
+        const float delta = grow ? mx : 0.f;
+        if (u > 0) {
+          const float alpha = fast_exp2(-delta);
+          l_run *= alpha;
+#pragma unroll
+          for (int db = 0; db < 4; ++db) O[db] *= alpha;
+        }
+        m_ref += delta;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) Cm[i] = kRaw ? -m_ref * inv_c : -m_ref;
+        const float dS = kRaw ? delta * inv_c : delta;
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) S[kk][r] -= dS;
+        lt = exp_tiles<kRaw>(S, Pf, c);
+      }
+    }
+    const int L0 = count(lm, 0);
+    if (__builtin_expect(L0 == count(lm, 3), 1)) {  // one level count (they do not decrease along the blocks)
+      switch (L0) {
+        case 8: qk_stream_copy<8>(kb, f, Qf, Cm, S, hook_qk); break;
+        case 7: qk_stream_copy<7>(kb, f, Qf, Cm, S, hook_qk); break;
+        case 6: qk_stream_copy<6>(kb, f, Qf, Cm, S, hook_qk); break;
+        case 5: qk_stream_copy<5>(kb, f, Qf, Cm, S, hook_qk); break;
+        case 4: qk_stream_copy<4>(kb, f, Qf, Cm, S, hook_qk); break;
+        case 3: qk_stream_copy<3>(kb, f, Qf, Cm, S, hook_qk); break;
+        case 2: qk_stream_copy<2>(kb, f, Qf, Cm, S, hook_qk); break;
+        default: qk_stream_copy<1>(kb, f, Qf, Cm, S, hook_qk); break;
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < 8; ++r) hook_qk(r);
+      qk_blocks(lm, kb, Qf, Cm, S);
+    }
+    l_run += lt;
+    // V of pair u and K of pair u + 2 have landed (K of u + 3, this wave's last 8
+    // loads, may still be in flight)
+    __builtin_amdgcn_s_waitcnt(kWaitVm | 8);
+    if ((2 * u + 2) * kPfTileN > a.nk) {
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh) {
+        const int n0 = (2 * u + hh) * kPfTileN + wave * kPage;
+        lds_u8* vpage = smem + kPfVRegion + (u & 1) * kPfPairBytes + hh * kPfSlotBytes + wave * 4096;
+#pragma unroll
+        for (int rr = 0; rr < 2; ++rr)
+#pragma unroll
+          for (int tk = 0; tk < kPage; ++tk)
+            if (n0 + tk >= a.nk)
+              *reinterpret_cast<__attribute__((address_space(3))) uint16_t*>(vpage + v_lds_elem(lane * 2 + rr, v_slot(tk))) =
+                  0;
+      }
+    }
+    pf_barrier();
+  }
+  // PV of the last pair
+  {
+    const lds_u8* vb = smem + kPfVRegion + ((U + 1) & 1) * kPfPairBytes + v_lane;
+    bf16x8 f[kRing];
+    pv_prefetch(vb, f);
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+      if (i + kRing - 1 < 32) f[(i + kRing - 1) % kRing] = lds_frag(stream_src(vb, vb, i + kRing - 1));
+      __builtin_amdgcn_sched_barrier(0);
+      O[i & 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[i % kRing], Pf[i >> 2], O[i & 3], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+
+  const float l = pair_sum(l_run);
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  if (row < a.nq) {
+    uint16_t* orow = a.out + static_cast<int64_t>(b) * a.o_sb + static_cast<int64_t>(row) * a.o_st +
+                     static_cast<int64_t>(h) * a.o_sh;
+#pragma unroll
+    for (int db = 0; db < 4; ++db) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int d = 32 * db + 8 * g + 4 * (lane >> 5);
+        u32x2 w;
+        w[0] = pack_bf16x2(O[db][4 * g + 0] * inv, O[db][4 * g + 1] * inv);
+        w[1] = pack_bf16x2(O[db][4 * g + 2] * inv, O[db][4 * g + 3] * inv);
+        *reinterpret_cast<u32x2*>(orow + d) = w;
+      }
+    }
+    if (a.lse != nullptr && lane < 32) {
+      a.lse[(static_cast<int64_t>(b) * a.hq + h) * a.nq + row] =
+          (l > 0.f) ? m_ref * kLn2 + __logf(l) : NEG_INF;
+    }
+  }
+}
+
 // ---- measurement probe: the MFMA ceiling of this kernel's structure ----
 // A pseudo-random bf16 value in about [-2, 2] (or [0, 1] for P), from a hash,
 // so that the matrix core switches as much as on real data (the part's power
@@ -904,6 +1316,8 @@ hipError_t ensure_lds_attribute() {
   if (g_attr_set[dev]) return hipSuccess;
   for (const void* f : {reinterpret_cast<const void*>(prefill_kernel<false>),
                         reinterpret_cast<const void*>(prefill_kernel<true>),
+                        reinterpret_cast<const void*>(prefill_solo_kernel<false>),
+                        reinterpret_cast<const void*>(prefill_solo_kernel<true>),
                         reinterpret_cast<const void*>(prefill_mfma_probe_kernel)}) {
     e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kPfLdsTotal);
     if (e != hipSuccess) return e;
@@ -913,16 +1327,36 @@ hipError_t ensure_lds_attribute() {
 }
 }  // namespace
 
+// Workgroups of a launch with `rows` query rows each (prefill_block's grid, in
+// rounds of 8 units).
+static int64_t prefill_blocks(const PrefillArgs& a, int rows) {
+  const int64_t units = static_cast<int64_t>((a.nq + rows - 1) / rows) * a.batch * a.hkv;
+  return (units + 7) / 8 * 8 * a.group;
+}
+
 hipError_t launch_prefill(const PrefillArgs& a, hipStream_t s) {
   if (a.nq <= 0 || a.batch <= 0) return hipSuccess;
   if (hipError_t e = ensure_lds_attribute(); e != hipSuccess) return e;
-  const int64_t units = static_cast<int64_t>(a.n_qtiles) * a.batch * a.hkv;
-  const int64_t blocks = (units + 7) / 8 * 8 * a.group;
+  // One wave per SIMD where every 128-row workgroup gets a CU of its own: an
+  // XCD's 32 CUs hold its share of the units (whole groups of q heads).  Past
+  // that line a second round starts and the fuller workgroups win (28 / 4 heads,
+  // k = 2: 1024 queries behind 32K keys, 224 workgroups, 531 -> 431 us; 2048
+  // tokens, 448, 57 -> 56; 4096 tokens 127 -> 152).
+  PrefillArgs k = a;
+  const bool solo = prefill_blocks(a, kSoloRowsWg) <= 256;
+  const int rows = solo ? kSoloRowsWg : kPfRowsWg;
+  k.n_qtiles = (a.nq + rows - 1) / rows;
+  const int64_t blocks = prefill_blocks(a, rows);
   if (blocks > INT32_MAX) return hipErrorInvalidConfiguration;
-  if (a.rope_cs != nullptr)
-    hipLaunchKernelGGL(prefill_kernel<false>, dim3(blocks), dim3(kPfWaves * 64), kPfLdsTotal, s, a);
-  else
-    hipLaunchKernelGGL(prefill_kernel<true>, dim3(blocks), dim3(kPfWaves * 64), kPfLdsTotal, s, a);
+#define ATF_PF_LAUNCH(K, W) hipLaunchKernelGGL(K, dim3(blocks), dim3((W) * 64), kPfLdsTotal, s, k)
+  if (solo) {
+    if (a.rope_cs != nullptr) ATF_PF_LAUNCH(prefill_solo_kernel<false>, kSoloWaves);
+    else ATF_PF_LAUNCH(prefill_solo_kernel<true>, kSoloWaves);
+  } else {
+    if (a.rope_cs != nullptr) ATF_PF_LAUNCH(prefill_kernel<false>, kPfWaves);
+    else ATF_PF_LAUNCH(prefill_kernel<true>, kPfWaves);
+  }
+#undef ATF_PF_LAUNCH
   return hipGetLastError();
 }
 
