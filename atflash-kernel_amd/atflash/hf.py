@@ -318,10 +318,10 @@ class WindowAttention:
                 raise ValueError("the cache was made for the other RoPE mode of this hook")
             if L == 1:
                 zhi = self.window.decode_zhi8 if windowed else None
-                o = ops.decode_paged(query[:, :, 0, :], lyr.kv, owner.page_table, owner.seq_lens(S), S, zhi,
+                o = ops.decode_paged(query.select(2, 0), lyr.kv, owner.page_table, owner.seq_lens(S), S, zhi,
                                      scale, owner.rope_cs, _lib.LAYOUT_HALF_SPLIT)
                 return o.view(b, 1, hq, d), None
-            zhi = list(self.window.prefill_zhi) if windowed else None
+            zhi = self.window.prefill_zhi if windowed else None
             o, _ = ops.prefill(query.transpose(1, 2), lyr.kv, owner.page_table, S, lyr.prev_length, zhi, scale,
                                owner.rope_cs, _lib.LAYOUT_HALF_SPLIT)
             return o, None  # [b, L, hq, d]

@@ -67,7 +67,10 @@ def pack_kv(k, v, rope=None, layout="half_split", start_pos=0):
     pages = -(-(int(start_pos) + N) // PAGE)
     kv_cache = torch.empty((B * pages, Hkv, *_lib.KV_BLOCK_SHAPE), dtype=torch.bfloat16, device=k.device)
     page_table = torch.arange(B * pages, dtype=torch.int32, device=k.device).view(B, pages)
-    starts = torch.full((B,), int(start_pos), dtype=torch.int32, device=k.device)
+    if B == 1 and start_pos == 0 and pages > 0:
+        starts = page_table[0, :1]  # the table's first entry, 0: a launch less
+    else:
+        starts = torch.full((B,), int(start_pos), dtype=torch.int32, device=k.device)
     ops.kv_write(kv_cache, k, v, starts, page_table, rope, _layout_id(layout))
     return kv_cache, page_table
 

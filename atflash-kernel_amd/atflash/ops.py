@@ -27,7 +27,7 @@ from . import _lib
 
 def _need_gpu(*ts):
     for t in ts:
-        if t is not None and not t.is_cuda:
+        if not (t is None or t.is_cuda):
             raise ValueError("atflash ops run on the GPU only (got a tensor on %s)" % t.device)
 
 
@@ -48,7 +48,8 @@ def _check_cache(kv_cache):
 
 
 def _layout(layout: int) -> int:
-    _need(layout in (_lib.LAYOUT_HALF_SPLIT, _lib.LAYOUT_SORTED_PAIR), f"unknown layout {layout}")
+    if layout != _lib.LAYOUT_HALF_SPLIT and layout != _lib.LAYOUT_SORTED_PAIR:
+        raise ValueError(f"unknown layout {layout}")
     return layout
 
 
@@ -68,22 +69,30 @@ def kv_write(kv_cache: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     start_pos[b] + t) into the paged cache, rotating K with rope_cs."""
     _need_gpu(kv_cache, k, v, start_pos, page_table, rope_cs)
     _check_cache(kv_cache)
-    _need(k.dtype == torch.bfloat16 and v.dtype == torch.bfloat16, "k and v must be bf16")
-    _need(k.dim() == 4 and k.shape == v.shape and k.shape[-1] == _lib.HEAD_DIM,
-          "k and v must be [B, T, Hkv, 128] of equal shape")
-    _need(k.shape[2] == kv_cache.shape[1], "k heads must equal the cache's kv heads")
-    _need(k.stride(-1) == 1 and v.stride(-1) == 1, "last dim of k and v must be contiguous")
-    _need(start_pos.dtype == torch.int32 and start_pos.numel() == k.shape[0], "start_pos must be int32 [B]")
-    _need(page_table.dtype == torch.int32 and page_table.dim() == 2 and page_table.shape[0] == k.shape[0]
-          and page_table.is_contiguous(), "page_table must be contiguous int32 [B, max_pages]")
+    if k.dtype != torch.bfloat16 or v.dtype != torch.bfloat16:
+        raise ValueError("k and v must be bf16")
+    ks, pool = k.shape, kv_cache.shape
+    if len(ks) != 4 or v.shape != ks or ks[3] != _lib.HEAD_DIM:
+        raise ValueError("k and v must be [B, T, Hkv, 128] of equal shape")
+    B, T, hkv, _ = ks
+    if hkv != pool[1]:
+        raise ValueError("k heads must equal the cache's kv heads")
+    ks_b, ks_t, ks_h, ks_d = k.stride()
+    vs_b, vs_t, vs_h, vs_d = v.stride()
+    if ks_d != 1 or vs_d != 1:
+        raise ValueError("last dim of k and v must be contiguous")
+    if start_pos.dtype != torch.int32 or start_pos.numel() != B:
+        raise ValueError("start_pos must be int32 [B]")
+    ps = page_table.shape
+    if page_table.dtype != torch.int32 or len(ps) != 2 or ps[0] != B or not page_table.is_contiguous():
+        raise ValueError("page_table must be contiguous int32 [B, max_pages]")
     rope_cs, max_pos = _rope(rope_cs)
-    L = _lib.lib()
-    _lib.check(L.atf_kv_write_bf16(
-        _lib.ptr(kv_cache), kv_cache.shape[0], kv_cache.shape[1],
-        _lib.ptr(k), k.stride(0), k.stride(1), k.stride(2),
-        _lib.ptr(v), v.stride(0), v.stride(1), v.stride(2),
-        k.shape[0], k.shape[1], _lib.ptr(start_pos.contiguous()), _lib.ptr(page_table), page_table.shape[1],
-        _lib.ptr(rope_cs), max_pos, _layout(layout), _lib.stream_of(k.device)))
+    if not start_pos.is_contiguous():
+        start_pos = start_pos.contiguous()
+    _lib.check(_lib.lib().atf_kv_write_bf16(
+        kv_cache.data_ptr(), pool[0], pool[1], k.data_ptr(), ks_b, ks_t, ks_h, v.data_ptr(), vs_b, vs_t, vs_h,
+        B, T, start_pos.data_ptr(), page_table.data_ptr(), ps[1],
+        None if rope_cs is None else rope_cs.data_ptr(), max_pos, _layout(layout), _lib.stream_of(k.device)))
 
 
 _kv_write_op = torch.library.custom_op("atflash::kv_write", kv_write, mutates_args=("kv_cache",))
@@ -102,22 +111,26 @@ def prefill(q: torch.Tensor, kv_cache: torch.Tensor, page_table: torch.Tensor,
     [B, Nq, Hq, 128], lse fp32 [B, Hq, Nq])."""
     _need_gpu(q, kv_cache, page_table, rope_cs)
     _check_cache(kv_cache)
-    _need(q.dtype == torch.bfloat16 and q.dim() == 4 and q.shape[-1] == _lib.HEAD_DIM,
-          "q must be bf16 [B, Nq, Hq, 128]")
-    _need(q.stride(-1) == 1, "last dim of q must be contiguous")
-    _need(page_table.dtype == torch.int32 and page_table.dim() == 2 and page_table.shape[0] == q.shape[0]
-          and page_table.is_contiguous(), "page_table must be contiguous int32 [B, max_pages]")
-    B, Nq, Hq, _ = q.shape
+    qs = q.shape
+    if q.dtype != torch.bfloat16 or len(qs) != 4 or qs[3] != _lib.HEAD_DIM:
+        raise ValueError("q must be bf16 [B, Nq, Hq, 128]")
+    q_sb, q_st, q_sh, q_sd = q.stride()
+    if q_sd != 1:
+        raise ValueError("last dim of q must be contiguous")
+    B, Nq, Hq, D = qs
+    ps = page_table.shape
+    if page_table.dtype != torch.int32 or len(ps) != 2 or ps[0] != B or not page_table.is_contiguous():
+        raise ValueError("page_table must be contiguous int32 [B, max_pages]")
     rope_cs, max_pos = _rope(rope_cs)
-    out = torch.empty((B, Nq, Hq, _lib.HEAD_DIM), dtype=torch.bfloat16, device=q.device)
-    lse = torch.empty((B, Hq, Nq), dtype=torch.float32, device=q.device)
-    L = _lib.lib()
-    _lib.check(L.atf_prefill_bf16(
-        _lib.ptr(out), out.stride(0), out.stride(1), out.stride(2), _lib.ptr(lse),
-        _lib.ptr(q), q.stride(0), q.stride(1), q.stride(2),
-        _lib.ptr(kv_cache), kv_cache.shape[0], _lib.ptr(page_table), page_table.shape[1],
-        B, Nq, int(nk), int(q_offset), Hq, kv_cache.shape[1], _lib.zhi_array(zhi), float(sm_scale),
-        _lib.ptr(rope_cs), max_pos, _layout(layout), _lib.stream_of(q.device)))
+    dev = q.device
+    out = torch.empty((B, Nq, Hq, D), dtype=torch.bfloat16, device=dev)
+    lse = torch.empty((B, Hq, Nq), dtype=torch.float32, device=dev)
+    pool = kv_cache.shape
+    _lib.check(_lib.lib().atf_prefill_bf16(
+        out.data_ptr(), Nq * Hq * D, Hq * D, D, lse.data_ptr(), q.data_ptr(), q_sb, q_st, q_sh,
+        kv_cache.data_ptr(), pool[0], page_table.data_ptr(), ps[1],
+        B, Nq, int(nk), int(q_offset), Hq, pool[1], _lib.zhi_array(zhi), float(sm_scale),
+        None if rope_cs is None else rope_cs.data_ptr(), max_pos, _layout(layout), _lib.stream_of(dev)))
     return out, lse
 
 
@@ -185,14 +198,17 @@ def decode_paged(q: torch.Tensor, kv_cache: torch.Tensor, page_table: torch.Tens
     _need_gpu(q, kv_cache, page_table, seq_lens, rope_cs)
     _check_cache(kv_cache)
     qs = q.shape
-    _need(q.dtype == torch.bfloat16 and len(qs) == 3 and qs[2] == _lib.HEAD_DIM, "q must be bf16 [B, Hq, 128]")
+    if q.dtype != torch.bfloat16 or len(qs) != 3 or qs[2] != _lib.HEAD_DIM:
+        raise ValueError("q must be bf16 [B, Hq, 128]")
     q_sb, q_sh, q_sd = q.stride()
-    _need(q_sd == 1, "last dim of q must be contiguous")
-    B, Hq = qs[0], qs[1]
-    _need(seq_lens.dtype == torch.int32 and seq_lens.numel() == B, "seq_lens must be int32 [B]")
+    if q_sd != 1:
+        raise ValueError("last dim of q must be contiguous")
+    B, Hq, _ = qs
+    if seq_lens.dtype != torch.int32 or seq_lens.numel() != B:
+        raise ValueError("seq_lens must be int32 [B]")
     ps = page_table.shape
-    _need(page_table.dtype == torch.int32 and len(ps) == 2 and ps[0] == B and page_table.is_contiguous(),
-          "page_table must be contiguous int32 [B, max_pages]")
+    if page_table.dtype != torch.int32 or len(ps) != 2 or ps[0] != B or not page_table.is_contiguous():
+        raise ValueError("page_table must be contiguous int32 [B, max_pages]")
     ks = kv_cache.shape
     num_pages, hkv = ks[0], ks[1]
     rope_cs, max_pos = _rope(rope_cs)
@@ -210,7 +226,7 @@ def decode_paged(q: torch.Tensor, kv_cache: torch.Tensor, page_table: torch.Tens
         out.data_ptr(), Hq * _lib.HEAD_DIM, _lib.HEAD_DIM, q.data_ptr(), q_sb, q_sh,
         kv_cache.data_ptr(), num_pages, page_table.data_ptr(), ps[1],
         seq_lens.data_ptr(), B, Hq, hkv, int(max_seq_len), table, float(sm_scale),
-        _lib.ptr(rope_cs), max_pos, _layout(layout), ws[0], ws[1], stream))
+        None if rope_cs is None else rope_cs.data_ptr(), max_pos, _layout(layout), ws[0], ws[1], stream))
     return out
 
 
@@ -249,7 +265,7 @@ def decode_rows(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, zhi, sm_scale
     _lib.check(L.atf_decode_rows_bf16(
         out.data_ptr(), Hq * _lib.HEAD_DIM, _lib.HEAD_DIM, q.data_ptr(), q_sb, q_sh,
         k.data_ptr(), kst[0], kst[1], kst[2], v.data_ptr(), vst[0], vst[1], vst[2],
-        B, Hq, hkv, N, _table(zhi, n), n, float(sm_scale), _lib.ptr(rope_cs), max_pos, _layout(layout),
+        B, Hq, hkv, N, _lib.zhi_array(zhi, n), n, float(sm_scale), _lib.ptr(rope_cs), max_pos, _layout(layout),
         ws[0], ws[1], stream))
     return out
 
