@@ -197,8 +197,8 @@ hipError_t launch_kv_write(const KvWriteArgs& a, hipStream_t s) {
   const int pages = (a.n_tokens + kPage - 1) / kPage + 1;
   // Heads per workgroup, by the call's token x head rows: few rows are spread over
   // more workgroups (517 tokens x 4 heads: kernel 8.1 us with four heads, 5.6 two,
-  // 4.8 one; 8192 x 8: call 17.2, 15.6, 17.2); many share the (cos, sin) rows
-  // 35.0); many share the (cos, sin) rows (128K x 4: 115.9, 123.3, 133.0).
+  // 4.8 one; calls on fresh buffers: 8192 x 8 17.0, 15.8, 17.2; 16K x 8 33.6,
+  // 33.0, 35.0); many share the (cos, sin) rows (128K x 4: 115.9, 123.3, 133.0).
   const int64_t rows = static_cast<int64_t>(a.n_tokens) * a.batch * a.hkv;
   if (rows <= 32 * 1024 || a.hkv == 1)
     hipLaunchKernelGGL(kv_write_kernel<1>, dim3(pages, a.batch, a.hkv), dim3(128), 0, s, a);

@@ -870,18 +870,32 @@ __device__ __forceinline__ void qk_stream_copy(const lds_u8* kb, bf16x8 (&f)[kRi
 }
 
 // S of the four 32-key blocks of a pair with a level count of its own each
-// (byte j of lm): one chain per block, a runtime loop over its levels.
+// (byte j of lm; not decreasing along the blocks): four interleaved chains, the
+// operands of level l + 1 read while level l's MFMAs run.
 __device__ __forceinline__ void qk_blocks(uint64_t lm, const lds_u8* kb, const u32x4 (&Qf)[kLevels], const f32x16& C,
                                           f32x16 (&S)[4]) {
+  bf16x8 f[4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const uint32_t m = (static_cast<uint32_t>(lm >> (8 * j)) & 0xffu) | 1u;  // levels as bits 0..L-1 (table order)
-    S[j] = C;
+  for (int j = 0; j < 4; ++j) f[j] = lds_frag(kb + j * 8192);
 #pragma unroll
-    for (int l = 0; l < kLevels; ++l)
-      if ((m >> l) & 1u)
-        S[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lds_frag(kb + j * 8192 + l * 512),
-                                                       __builtin_bit_cast(bf16x8, Qf[l]), S[j], 0, 0, 0);
+  for (int l = 0; l < kLevels; ++l) {
+    // level l of block j is read iff bit 8j + l of lm is set, level 0 always
+    bf16x8 n[4];
+    const bool more = l + 1 < kLevels && ((lm >> (24 + l + 1)) & 1u) != 0;
+    if (more) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) n[j] = lds_frag(kb + j * 8192 + (l + 1) * 512);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (l == 0 || ((lm >> (8 * j + l)) & 1u) != 0)
+        S[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[j], __builtin_bit_cast(bf16x8, Qf[l]), l == 0 ? C : S[j], 0, 0,
+                                                       0);
+    __builtin_amdgcn_sched_barrier(0);
+    if (!more) break;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) f[j] = n[j];
   }
 }
 
@@ -939,7 +953,10 @@ void prefill_solo_kernel(PrefillArgs a) {
   int tab_n = fetch64(1);
   int tab_v = tab_k;
 
+  // Q and its (cos, sin) rows are requested here and used after the K copies are
+  // on their way: one memory round trip for all of them.
   u32x4 Qf[kLevels];
+  float cs[kLevels][8];
   const bool second = lane >= 32;
   const int row = lr0 + (lane & 31);
   {
@@ -949,17 +966,13 @@ void prefill_solo_kernel(PrefillArgs a) {
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       u32x4 v[4];
-      const int s0 = 8 * j + (second ? 1 : 0);
-      load_slices4<2>(qrow, a.layout, s0, v);
-      if (a.rope_cs != nullptr) {
-        float cs[4][8];
+      load_slices4<2>(qrow, a.layout, 8 * j + (second ? 1 : 0), v);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) load_cs4(a.rope_cs, a.q_offset + row_c, slice_pair0(s0 + 2 * i), cs[i]);
+      for (int i = 0; i < 4; ++i) Qf[4 * j + i] = v[i];
+    }
+    if (a.rope_cs != nullptr) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = rope_slice(v[i], cs[i], a.scale_log2);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) Qf[4 * j + i] = (row < a.nq) ? v[i] : u32x4{0u, 0u, 0u, 0u};
+      for (int i = 0; i < kLevels; ++i) load_cs4(a.rope_cs, a.q_offset + row_c, slice_pair0(2 * i + (second ? 1 : 0)), cs[i]);
     }
   }
 
@@ -1021,6 +1034,11 @@ void prefill_solo_kernel(PrefillArgs a) {
     const PageCopy c0 = k_page(p, 0, (count(lm, 4) + 1) >> 1), c1 = k_page(p, 1, (count(lm, 5) + 1) >> 1);
 #pragma unroll
     for (int r = 0; r < 8; ++r) copy_row_n(r < 4 ? c0 : c1, k_off, r & 3);
+  }
+#pragma unroll
+  for (int i = 0; i < kLevels; ++i) {
+    if (a.rope_cs != nullptr) Qf[i] = rope_slice(Qf[i], cs[i], a.scale_log2);
+    if (row >= a.nq) Qf[i] = u32x4{0u, 0u, 0u, 0u};
   }
   // V pair 1: read by the first PV with P = 0
   zero_page(smem + kPfVRegion + kPfPairBytes + wave * 4096, lane);
