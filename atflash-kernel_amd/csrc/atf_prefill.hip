@@ -879,13 +879,12 @@ __device__ __forceinline__ void qk_blocks(uint64_t lm, const lds_u8* kb, const u
   for (int j = 0; j < 4; ++j) f[j] = lds_frag(kb + j * 8192);
 #pragma unroll
   for (int l = 0; l < kLevels; ++l) {
-    // level l of block j is read iff bit 8j + l of lm is set, level 0 always
+    // level l of block j is read iff bit 8j + l of lm is set, level 0 always; an
+    // operand past the levels is read ahead and not used (its address is inside
+    // the staged pair)
     bf16x8 n[4];
-    const bool more = l + 1 < kLevels && ((lm >> (24 + l + 1)) & 1u) != 0;
-    if (more) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) n[j] = lds_frag(kb + j * 8192 + (l + 1) * 512);
-    }
+    for (int j = 0; j < 4; ++j) n[j] = l + 1 < kLevels ? lds_frag(kb + j * 8192 + (l + 1) * 512) : f[j];
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < 4; ++j)
@@ -893,7 +892,6 @@ __device__ __forceinline__ void qk_blocks(uint64_t lm, const lds_u8* kb, const u
         S[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[j], __builtin_bit_cast(bf16x8, Qf[l]), l == 0 ? C : S[j], 0, 0,
                                                        0);
     __builtin_amdgcn_sched_barrier(0);
-    if (!more) break;
 #pragma unroll
     for (int j = 0; j < 4; ++j) f[j] = n[j];
   }
