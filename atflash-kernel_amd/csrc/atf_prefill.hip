@@ -451,6 +451,105 @@ __device__ __forceinline__ float exp_tiles(const f32x16 (&S)[4], bf16x8 (&Pf)[8]
   return lt;
 }
 
+// ---- Q in, O out: whole rows through LDS ----
+// A fragment holds 16 bytes of each of 32 rows, so reading Q and (cos, sin) as
+// fragments, or storing O from its accumulators, touches 32 rows with 8 to 32
+// bytes of each an instruction; the vector memory path takes such an instruction
+// line by line, 48 of them a wave (a 256-row workgroup's 192 KB of Q and (cos,
+// sin) lines do not stay in the 32 KB L1 between them).  Instead 8 lanes (Q) or
+// 16 (O) take a row's whole lines, and a wave turns rows into fragments, or back,
+// in 8 KB of LDS of its own that no copy uses at that time.
+//   24 / 8 heads, OFF: 8 x 700 tokens 81.5 -> 66 us, 8 x 256 26 -> 20, 64 x 256
+// 152 -> 121; 28 / 4 heads, k = 2: 2048 tokens 56.5 -> 51, 4096 128 -> 120, 32768
+// 5.22 -> 5.16 ms; 128 tokens 13.6 -> 10.9.  A launch of one or two waves pays the
+// LDS round trips instead: up to 32 tokens 11.1 -> 11.7.
+constexpr int kRowStage = 32 * 2 * kP * 2;           // 32 rows, 8 KB a wave
+typedef u32x4 u32x4_a8 __attribute__((aligned(8)));    // `out` is 8-byte aligned
+
+// 32 rows of Q as requested: lane 8k + j holds, of rows 8i + k (i = 0..3), rotary
+// pairs 8j .. 8j+7 (slices 14 - 2j and 15 - 2j) with their (cos, sin).
+struct QRows {
+  u32x4 x[4][2];
+  float cs[4][16];
+};
+
+// Rows past nq read row nq - 1, in bounds.
+__device__ __forceinline__ void q_request(const PrefillArgs& a, int b, int h, int lr0, int lane, QRows& q) {
+  const int j = lane & 7;
+  const bool half = a.layout == kLayoutHalfSplit;
+  const int c0 = half ? 8 * j : 8 * (14 - 2 * j), c1 = half ? kP + 8 * j : 8 * (15 - 2 * j);
+  const uint16_t* qh = a.q + static_cast<int64_t>(b) * a.q_sb + static_cast<int64_t>(h) * a.q_sh;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint16_t* qrow = qh + static_cast<int64_t>(min(lr0 + 8 * i + (lane >> 3), a.nq - 1)) * a.q_st;
+    q.x[i][0] = ldg16(qrow + c0);
+    q.x[i][1] = ldg16(qrow + c1);
+  }
+  if (a.rope_cs != nullptr) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      load_cs8(a.rope_cs, a.q_offset + min(lr0 + 8 * i + (lane >> 3), a.nq - 1), 8 * j, q.cs[i]);
+  }
+}
+
+// The requested rows, rotated and scaled, as the wave's B operands (read before
+// the caller's barrier, after which copies may reuse `st`): k half h of
+// level l is slice 2l + h, as in the cache's K pages.  Slice s of row r lies at
+// 512 s + 16 (r ^ 8 (s/2 % 4)): the 8 rows x 8 slices of a write, and the 32 rows
+// of a read, spread over all banks.
+__device__ __forceinline__ void q_fragments(const PrefillArgs& a, const QRows& q, lds_u8* st, int lr0, int lane,
+                                            u32x4 (&Qf)[kLevels]) {
+  const int j = lane & 7;
+  const bool half = a.layout == kLayoutHalfSplit;
+  auto at = [&](int s, int r) {
+    return reinterpret_cast<__attribute__((address_space(3))) u32x4*>(st + 512 * s + 16 * (r ^ (((s >> 1) & 3) << 3)));
+  };
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const u32x4 x0 = q.x[i][0], x1 = q.x[i][1];
+    u32x4 lo = half ? u32x4{x0[2], x0[3], x1[2], x1[3]} : x0;  // slice 14 - 2j: pairs 8j+4 .. 8j+7
+    u32x4 hi = half ? u32x4{x0[0], x0[1], x1[0], x1[1]} : x1;  // slice 15 - 2j: pairs 8j .. 8j+3
+    if (a.rope_cs != nullptr) {
+      lo = rope_slice(lo, q.cs[i] + 8, a.scale_log2);
+      hi = rope_slice(hi, q.cs[i], a.scale_log2);
+    }
+    const int r = 8 * i + (lane >> 3);
+    *at(14 - 2 * j, r) = lo;
+    *at(15 - 2 * j, r) = hi;
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave's own writes, read by its other lanes
+#pragma unroll
+  for (int l = 0; l < kLevels; ++l) {
+    const u32x4 v = *at(2 * l + (lane >> 5), lane & 31);
+    Qf[l] = (lr0 + (lane & 31) < a.nq) ? v : u32x4{0u, 0u, 0u, 0u};
+  }
+}
+
+// O / l of the wave's 32 rows to memory.  In LDS row r is 256 bytes, its 16-byte
+// chunk c at c ^ (r % 16).
+__device__ __forceinline__ void store_rows(const PrefillArgs& a, int b, int h, int lr0, int lane, const f32x16 (&O)[4],
+                                           float inv, lds_u8* st) {
+  const int r = lane & 31;
+#pragma unroll
+  for (int db = 0; db < 4; ++db)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      u32x2 w;  // dims 32 db + 8 g + 4 (lane / 32) .. + 3
+      w[0] = pack_bf16x2(O[db][4 * g + 0] * inv, O[db][4 * g + 1] * inv);
+      w[1] = pack_bf16x2(O[db][4 * g + 2] * inv, O[db][4 * g + 3] * inv);
+      *reinterpret_cast<__attribute__((address_space(3))) u32x2*>(st + 256 * r + 16 * ((4 * db + g) ^ (r & 15)) +
+                                                                  8 * (lane >> 5)) = w;
+    }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  uint16_t* oh = a.out + static_cast<int64_t>(b) * a.o_sb + static_cast<int64_t>(h) * a.o_sh + 8 * (lane & 15);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int rr = 4 * i + (lane >> 4);
+    const u32x4 w = *reinterpret_cast<__attribute__((address_space(3))) u32x4*>(st + 256 * rr + 16 * ((lane ^ rr) & 15));
+    if (lr0 + rr < a.nq) *reinterpret_cast<u32x4_a8*>(oh + static_cast<int64_t>(lr0 + rr) * a.o_st) = w;
+  }
+}
+
 // Block -> (sequence, q head, query tile), XCD-aware: block i runs on XCD i % 8
 // (were it not so, that would cost time, not results).  The units (query tile,
 // sequence, kv head), heaviest (last) tiles first, are dealt out one to an XCD in
@@ -511,35 +610,12 @@ __global__ __launch_bounds__(kPfWaves * 64, 1) void prefill_kernel(PrefillArgs a
   const int t_end =
       (lr0 < a.nq) ? min(n_ktiles, (a.q_offset + min(a.nq, lr0 + kPfRowsWave) - 1) / kPfTileN + 1) : 0;
 
-  // ---- Q fragments (B operand of S^T = K Q^T), with RoPE and the log2-unit
-  // softmax scale applied at load ----
-  // Every Q and (cos, sin) load is issued before any is used, four levels at a
-  // time (one memory round trip per four levels instead of one per level):
-  // rows past nq read row nq - 1, in bounds, and are zeroed afterwards.
+  // Q (B operand of S^T = K Q^T), with RoPE and the log2-unit softmax scale
+  // applied at load: requested here, made into fragments behind the first K copies.
   u32x4 Qf[kLevels];
-  const bool second = lane >= 32;
   const int row = lr0 + (lane & 31);
-  {
-    const int row_c = min(row, a.nq - 1);
-    const uint16_t* qrow = a.q + static_cast<int64_t>(b) * a.q_sb + static_cast<int64_t>(row_c) * a.q_st +
-                           static_cast<int64_t>(h) * a.q_sh;
-    // k half h of level l is slice 2l + h, as in the cache's K pages
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      u32x4 v[4];
-      const int s0 = 8 * j + (second ? 1 : 0);  // levels 4j .. 4j+3: slices s0, s0+2, s0+4, s0+6
-      load_slices4<2>(qrow, a.layout, s0, v);
-      if (a.rope_cs != nullptr) {
-        float cs[4][8];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) load_cs4(a.rope_cs, a.q_offset + row_c, slice_pair0(s0 + 2 * i), cs[i]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = rope_slice(v[i], cs[i], a.scale_log2);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) Qf[4 * j + i] = (row < a.nq) ? v[i] : u32x4{0u, 0u, 0u, 0u};
-    }
-  }
+  QRows q;
+  q_request(a, b, h, lr0, lane, q);
 
   f32x16 O[4];
 #pragma unroll
@@ -587,6 +663,8 @@ __global__ __launch_bounds__(kPfWaves * 64, 1) void prefill_kernel(PrefillArgs a
         *reinterpret_cast<__attribute__((address_space(3))) u32x4*>(
             smem + kPfVRegion + kPfPairBytes + s * kPfSlotBytes + rank * 4096 + i * 1024 + lane * 16) = z;
   }
+  // staged in K pairs 1 and 2, which are copied to after the barrier
+  q_fragments(a, q, smem + kPfPairBytes + wave * kRowStage, lr0, lane, Qf);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (!copies_v) {
@@ -782,25 +860,10 @@ __global__ __launch_bounds__(kPfWaves * 64, 1) void prefill_kernel(PrefillArgs a
   // ---- epilogue: normalise and store ----
   const float l = pair_sum(l_run);
   const float inv = l > 0.f ? 1.f / l : 0.f;
-  if (row < a.nq) {
-    uint16_t* orow = a.out + static_cast<int64_t>(b) * a.o_sb + static_cast<int64_t>(row) * a.o_st +
-                     static_cast<int64_t>(h) * a.o_sh;
-#pragma unroll
-    for (int db = 0; db < 4; ++db) {
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int d = 32 * db + 8 * g + 4 * (lane >> 5);
-        u32x2 w;
-        w[0] = pack_bf16x2(O[db][4 * g + 0] * inv, O[db][4 * g + 1] * inv);
-        w[1] = pack_bf16x2(O[db][4 * g + 2] * inv, O[db][4 * g + 3] * inv);
-        *reinterpret_cast<u32x2*>(orow + d) = w;
-      }
-    }
-    if (a.lse != nullptr && lane < 32) {
-      a.lse[(static_cast<int64_t>(b) * a.hq + h) * a.nq + row] =
-          (l > 0.f) ? m_ref * kLn2 + __logf(l) : NEG_INF;
-    }
-  }
+  // (no wave reads a K pair past the last barrier, and every copy has landed)
+  store_rows(a, b, h, lr0, lane, O, inv, smem + wave * kRowStage);
+  if (a.lse != nullptr && lane < 32 && row < a.nq)
+    a.lse[(static_cast<int64_t>(b) * a.hq + h) * a.nq + row] = (l > 0.f) ? m_ref * kLn2 + __logf(l) : NEG_INF;
 }
 
 // ---- one wave per SIMD: launches that leave CUs idle ----
@@ -954,25 +1017,9 @@ void prefill_solo_kernel(PrefillArgs a) {
   // Q and its (cos, sin) rows are requested here and used after the K copies are
   // on their way: one memory round trip for all of them.
   u32x4 Qf[kLevels];
-  float cs[kLevels][8];
-  const bool second = lane >= 32;
   const int row = lr0 + (lane & 31);
-  {
-    const int row_c = min(row, a.nq - 1);
-    const uint16_t* qrow = a.q + static_cast<int64_t>(b) * a.q_sb + static_cast<int64_t>(row_c) * a.q_st +
-                           static_cast<int64_t>(h) * a.q_sh;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      u32x4 v[4];
-      load_slices4<2>(qrow, a.layout, 8 * j + (second ? 1 : 0), v);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) Qf[4 * j + i] = v[i];
-    }
-    if (a.rope_cs != nullptr) {
-#pragma unroll
-      for (int i = 0; i < kLevels; ++i) load_cs4(a.rope_cs, a.q_offset + row_c, slice_pair0(2 * i + (second ? 1 : 0)), cs[i]);
-    }
-  }
+  QRows q;
+  q_request(a, b, h, lr0, lane, q);
 
   f32x16 O[4];
 #pragma unroll
@@ -1033,11 +1080,8 @@ void prefill_solo_kernel(PrefillArgs a) {
 #pragma unroll
     for (int r = 0; r < 8; ++r) copy_row_n(r < 4 ? c0 : c1, k_off, r & 3);
   }
-#pragma unroll
-  for (int i = 0; i < kLevels; ++i) {
-    if (a.rope_cs != nullptr) Qf[i] = rope_slice(Qf[i], cs[i], a.scale_log2);
-    if (row >= a.nq) Qf[i] = u32x4{0u, 0u, 0u, 0u};
-  }
+  // staged in V pair 0, which is copied to after the barrier
+  q_fragments(a, q, smem + kPfVRegion + wave * kRowStage, lr0, lane, Qf);
   // V pair 1: read by the first PV with P = 0
   zero_page(smem + kPfVRegion + kPfPairBytes + wave * 4096, lane);
   zero_page(smem + kPfVRegion + kPfPairBytes + kPfSlotBytes + wave * 4096, lane);
@@ -1176,25 +1220,11 @@ void prefill_solo_kernel(PrefillArgs a) {
 
   const float l = pair_sum(l_run);
   const float inv = l > 0.f ? 1.f / l : 0.f;
-  if (row < a.nq) {
-    uint16_t* orow = a.out + static_cast<int64_t>(b) * a.o_sb + static_cast<int64_t>(row) * a.o_st +
-                     static_cast<int64_t>(h) * a.o_sh;
-#pragma unroll
-    for (int db = 0; db < 4; ++db) {
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int d = 32 * db + 8 * g + 4 * (lane >> 5);
-        u32x2 w;
-        w[0] = pack_bf16x2(O[db][4 * g + 0] * inv, O[db][4 * g + 1] * inv);
-        w[1] = pack_bf16x2(O[db][4 * g + 2] * inv, O[db][4 * g + 3] * inv);
-        *reinterpret_cast<u32x2*>(orow + d) = w;
-      }
-    }
-    if (a.lse != nullptr && lane < 32) {
-      a.lse[(static_cast<int64_t>(b) * a.hq + h) * a.nq + row] =
-          (l > 0.f) ? m_ref * kLn2 + __logf(l) : NEG_INF;
-    }
-  }
+  // The V pair that the last barrier freed (the other one is read above; zeros past
+  // the end may still land in a K pair).
+  store_rows(a, b, h, lr0, lane, O, inv, smem + kPfVRegion + (U & 1) * kPfPairBytes + wave * kRowStage);
+  if (a.lse != nullptr && lane < 32 && row < a.nq)
+    a.lse[(static_cast<int64_t>(b) * a.hq + h) * a.nq + row] = (l > 0.f) ? m_ref * kLn2 + __logf(l) : NEG_INF;
 }
 
 // ---- measurement probe: the MFMA ceiling of this kernel's structure ----
