@@ -561,7 +561,7 @@ __device__ __forceinline__ void store_rows(const PrefillArgs& a, int b, int h, i
 //   Dealing out whole query tiles instead (all heads of a tile on one XCD, one
 // sequence after the other) left XCDs without work below 8 tiles a sequence,
 // whatever the batch: 8 x 700 tokens of 24 heads ran on 3 of 8 XCDs, 191 us
-// against 82 here; 1024 queries behind 32K keys (28 heads) on 4, 649 against
+// against 82 (both before Q and O moved in whole rows); 1024 queries behind 32K keys (28 heads) on 4, 649 against
 // 531; 4 x 2048 tokens 237 against 172; 5000 tokens 197 against 187.  At 32K
 // tokens and up the two are within 1% (28 / 4 heads, windowed 128K 75.9 ms
 // against 75.6), 4% in favour of this one with 24 / 8 heads (68.6 against 65.9);
@@ -610,13 +610,6 @@ __global__ __launch_bounds__(kPfWaves * 64, 1) void prefill_kernel(PrefillArgs a
   const int t_end =
       (lr0 < a.nq) ? min(n_ktiles, (a.q_offset + min(a.nq, lr0 + kPfRowsWave) - 1) / kPfTileN + 1) : 0;
 
-  // Q (B operand of S^T = K Q^T), with RoPE and the log2-unit softmax scale
-  // applied at load: requested here, made into fragments behind the first K copies.
-  u32x4 Qf[kLevels];
-  const int row = lr0 + (lane & 31);
-  QRows q;
-  q_request(a, b, h, lr0, lane, q);
-
   f32x16 O[4];
 #pragma unroll
   for (int db = 0; db < 4; ++db) O[db] = f32x16{};
@@ -643,46 +636,47 @@ __global__ __launch_bounds__(kPfWaves * 64, 1) void prefill_kernel(PrefillArgs a
   const int v_lane = (lane >> 5) * 512 + (lane & 31) * 16;
 
   // ---- prologue ----
-  // Group 0 copies K, group 1 copies V, each wave page `rank` of a tile.  Group
-  // 0 stages the K of tiles 0 and 1 (waited for here) and requests tiles 2 and
-  // 3; group 1 zeroes V pair 1 (read with P = 0 by phase 0) and requests the V
-  // of tiles 0 and 1.  pg_a / pg_b: page-table entries of the wave's next two
-  // copies, fetched one phase ahead.
-  int pg_a, pg_b;
-  if (!copies_v) {
-    const int e0 = fetch_page(a, b, rank), e1 = fetch_page(a, b, 4 + rank);
-    const int p0 = page_id(a, e0), p1 = page_id(a, e1);
-    if (0 < T) pf_load_page(a, kvh, p0, w_ld.advance(a.lt, 0), false, smem + rank * 4096, lane, copy_off);
-    if (1 < T) pf_load_page(a, kvh, p1, w_ld.advance(a.lt, 1), false, smem + kPfSlotBytes + rank * 4096, lane, copy_off);
-  } else {
-    const u32x4 z = {0u, 0u, 0u, 0u};
+  // Group 0 copies K, group 1 copies V, each wave page `rank` of a tile.  Page-table
+  // entries first, then Q (B operand of S^T = K Q^T; RoPE and the log2-unit softmax
+  // scale are applied as it becomes fragments), then group 0 requests the K of tiles
+  // 0 to 3 and group 1 zeroes V pair 1 (read with P = 0 by phase 0): one wait for
+  // all of it.  Q is staged in K pair 2 and V pair 0, which are copied to behind the
+  // barrier: V of tiles 0 and 1 at once, K of tiles 4 and 5 in phase 0.
+  // With the entries behind Q and a second round trip for tiles 2 and 3 behind the
+  // barrier, a unit's start took 16500 cycles, of 43700 for 256 queries and keys:
+  // 8 x 700 tokens (24 / 8 heads) 66.0 -> 62.7 us, 4096 (28 / 4) 118.2 -> 117.2.
+  // pg_a / pg_b: page-table entries of the wave's next two copies, fetched one
+  // phase ahead.
+  int e[4], pg_a = 0, pg_b = 0;
 #pragma unroll
-    for (int s = 0; s < 2; ++s)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        *reinterpret_cast<__attribute__((address_space(3))) u32x4*>(
-            smem + kPfVRegion + kPfPairBytes + s * kPfSlotBytes + rank * 4096 + i * 1024 + lane * 16) = z;
-  }
-  // staged in K pairs 1 and 2, which are copied to after the barrier
-  q_fragments(a, q, smem + kPfPairBytes + wave * kRowStage, lr0, lane, Qf);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
+  for (int t = 0; t < 4; ++t) e[t] = fetch_page(a, b, 4 * t + rank);
   if (!copies_v) {
-    const int e2 = fetch_page(a, b, 8 + rank), e3 = fetch_page(a, b, 12 + rank);
-    const int p2 = page_id(a, e2), p3 = page_id(a, e3);
-    if (2 < T) pf_load_page(a, kvh, p2, w_ld.advance(a.lt, 2), false, smem + kPfPairBytes + rank * 4096, lane, copy_off);
-    if (3 < T)
-      pf_load_page(a, kvh, p3, w_ld.advance(a.lt, 3), false, smem + kPfPairBytes + kPfSlotBytes + rank * 4096, lane,
-                   copy_off);
     pg_a = fetch_page(a, b, 16 + rank);
     pg_b = fetch_page(a, b, 20 + rank);
+  }
+  u32x4 Qf[kLevels];
+  const int row = lr0 + (lane & 31);
+  QRows q;
+  q_request(a, b, h, lr0, lane, q);
+  if (!copies_v) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      if (t < T)
+        pf_load_page(a, kvh, page_id(a, e[t]), w_ld.advance(a.lt, t), false, smem + t * kPfSlotBytes + rank * 4096, lane,
+                     copy_off);
   } else {
-    const int e0 = fetch_page(a, b, rank), e1 = fetch_page(a, b, 4 + rank);
-    const int p0 = page_id(a, e0), p1 = page_id(a, e1);
-    if (0 < T2) pf_load_page(a, kvh, p0, kLevels, true, smem + kPfVRegion + rank * 4096, lane, copy_off);
-    if (1 < T2) pf_load_page(a, kvh, p1, kLevels, true, smem + kPfVRegion + kPfSlotBytes + rank * 4096, lane, copy_off);
-    pg_a = fetch_page(a, b, 8 + rank);
-    pg_b = fetch_page(a, b, 12 + rank);
+#pragma unroll
+    for (int s = 0; s < 2; ++s) zero_page(smem + kPfVRegion + kPfPairBytes + s * kPfSlotBytes + rank * 4096, lane);
+  }
+  q_fragments(a, q, smem + (copies_v ? kPfVRegion : 2 * kPfPairBytes) + rank * kRowStage, lr0, lane, Qf);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (copies_v) {
+    if (0 < T2) pf_load_page(a, kvh, page_id(a, e[0]), kLevels, true, smem + kPfVRegion + rank * 4096, lane, copy_off);
+    if (1 < T2)
+      pf_load_page(a, kvh, page_id(a, e[1]), kLevels, true, smem + kPfVRegion + kPfSlotBytes + rank * 4096, lane, copy_off);
+    pg_a = e[2];
+    pg_b = e[3];
     pf_barrier();  // group 1 starts one step late
   }
 
@@ -1257,8 +1251,9 @@ __device__ __forceinline__ u32x4 probe_vec(uint32_t seed, bool unit) {
                probe_bf16x2(probe_hash(seed * 4 + 2), unit), probe_bf16x2(probe_hash(seed * 4 + 3), unit)};
 }
 
-// The prefill kernel's MFMA work with nothing else: the same grid
-// (heaviest tiles first, serpentine over the XCDs), waves, tile-pair count per workgroup (causal, nk = nq, window OFF),
+// The prefill kernel's MFMA work with nothing else: its workgroups for one
+// sequence (heaviest tiles first, whole tiles dealt over the XCDs in alternating
+// order), waves, tile-pair count per workgroup (causal, nk = nq, window OFF),
 // LDS operand ring and stream order (PV of 8 pages then QK of 8 levels over
 // four 32-key blocks, 64 MFMAs per pair), s_setprio and the two barriers per
 // pair with the two wave groups one phase apart -- but no softmax, no K/V
