@@ -561,11 +561,11 @@ __device__ __forceinline__ void store_rows(const PrefillArgs& a, int b, int h, i
 //   Dealing out whole query tiles instead (all heads of a tile on one XCD, one
 // sequence after the other) left XCDs without work below 8 tiles a sequence,
 // whatever the batch: 8 x 700 tokens of 24 heads ran on 3 of 8 XCDs, 191 us
-// against 82 (both before Q and O moved in whole rows); 1024 queries behind 32K keys (28 heads) on 4, 649 against
-// 531; 4 x 2048 tokens 237 against 172; 5000 tokens 197 against 187.  At 32K
-// tokens and up the two are within 1% (28 / 4 heads, windowed 128K 75.9 ms
-// against 75.6), 4% in favour of this one with 24 / 8 heads (68.6 against 65.9);
-// outputs bitwise equal.
+// against 82 (both before Q and O moved in whole rows); 1024 queries behind 32K
+// keys (28 heads) on 4, 649 against 531; 4 x 2048 tokens 237 against 172; 5000
+// tokens 197 against 187.  At 32K tokens and up the two are within 1% (28 / 4
+// heads, windowed 128K 75.9 ms against 75.6), 4% in favour of this one with 24 /
+// 8 heads (68.6 against 65.9); outputs bitwise equal.
 __device__ __forceinline__ bool prefill_block(const PrefillArgs& a, int bid, int& b, int& h, int& qt) {
   const int xcd = bid & 7;
   const int j = bid >> 3;
