@@ -459,7 +459,7 @@ void decode_kernel(const int32_t* page_table, const int32_t* seq_lens, const uin
 // the beginning of another.  The lengths live in device memory, so every
 // workgroup derives its run from them (one load per 64 sequences, sums by DPP).
 // A sequence inside one run is written by its workgroup; a cut one leaves a
-// partial per run, merged by decode_merge_kernel<true>.  Run c's partials are 2c
+// partial per run, merged by decode_batch_merge_kernel.  Run c's partials are 2c
 // (of a sequence that it begins with) and 2c + 1 (of one that begins inside it).
 //   HBM bound.  Measured against decode_kernel on the same batch (24 / 8 heads,
 // vec8 k = 2; us a call): 12 sequences of 700 to 32768 tokens 110 -> 73, 16 of
@@ -1021,11 +1021,8 @@ __device__ __forceinline__ void merge_lane_groups(float& m, float& l, f32x4& o, 
 // kBatch: the partials of decode_batch_kernel (n_splits holds the runs per kv
 // head); a sequence in one run has its output already, an empty one is zeroed here.
 template <bool kBatch>
-__global__ __launch_bounds__(512) void decode_merge_kernel(const float* ws_ml, const float* ws_o, uint16_t* out,
-                                                            int64_t o_sb, int64_t o_sh, int n_splits, int group,
-                                                            int hkv, float scale_log2, const int32_t* seq_lens,
-                                                            int batch, int max_seq_len) {
-  MergeArgs a{ws_ml, ws_o, out, o_sb, o_sh, n_splits, group, hkv, scale_log2};
+__device__ __forceinline__ void merge_splits(MergeArgs a, const int32_t* seq_lens, int batch, int max_seq_len) {
+  const int n_splits = a.n_splits;
   const int chunk = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
   int64_t part0 = (static_cast<int64_t>(b) * a.hkv + h) * a.n_splits;  // split 0's partial
   int step = 1, skew = 0;  // split i's is part0 + step * i, less skew after the first
@@ -1112,6 +1109,24 @@ __global__ __launch_bounds__(512) void decode_merge_kernel(const float* ws_ml, c
   }
 }
 
+// The lengths are the batch kernel's own arguments: 56 bytes of arguments are one
+// line to write per launch, 72 are two, on a path where the host sets the time
+// (8K tokens, one sequence: 13.0 -> 11.5 to 12.0 us a call; 1003 by a plan: 10.3 ->
+// 9.1 to 10.1).
+__global__ __launch_bounds__(512) void decode_merge_kernel(const float* ws_ml, const float* ws_o, uint16_t* out,
+                                                           int64_t o_sb, int64_t o_sh, int n_splits, int group,
+                                                           int hkv, float scale_log2) {
+  merge_splits<false>(MergeArgs{ws_ml, ws_o, out, o_sb, o_sh, n_splits, group, hkv, scale_log2}, nullptr, 0, 0);
+}
+
+__global__ __launch_bounds__(512) void decode_batch_merge_kernel(const float* ws_ml, const float* ws_o, uint16_t* out,
+                                                                 int64_t o_sb, int64_t o_sh, int n_splits, int group,
+                                                                 int hkv, float scale_log2, const int32_t* seq_lens,
+                                                                 int batch, int max_seq_len) {
+  merge_splits<true>(MergeArgs{ws_ml, ws_o, out, o_sb, o_sh, n_splits, group, hkv, scale_log2}, seq_lens, batch,
+                     max_seq_len);
+}
+
 // Level count per page for one sequence of length N under the page rule
 // (block_n = 16), as page_slices<false> computes it (the kernel reads twice as
 // many 8-dim slices).
@@ -1124,14 +1139,16 @@ __global__ void decode_page_levels_kernel(int32_t* out, int n_pages, int N, Leve
 // The merge of a call's split partials (nothing to do with one split).
 static hipError_t launch_merge(const DecodeArgs& a, hipStream_t s) {
   const dim3 grid(kMergeChunks, a.hkv, a.batch);
-#define ATF_MERGE_LAUNCH(BATCH, N)                                                                                 \
-  hipLaunchKernelGGL(decode_merge_kernel<BATCH>, grid, dim3(512), 0, s, static_cast<const float*>(a.ws_ml),       \
-                     static_cast<const float*>(a.ws_o), a.out, a.o_sb, a.o_sh, N, a.group, a.hkv, a.scale_log2,   \
-                     a.seq_lens, a.batch, a.max_seq_len)
-  if (a.runs > 0) ATF_MERGE_LAUNCH(true, a.runs);
-  else if (a.n_splits > 1) ATF_MERGE_LAUNCH(false, a.n_splits);
-  else return hipSuccess;
-#undef ATF_MERGE_LAUNCH
+  if (a.runs > 0)
+    hipLaunchKernelGGL(decode_batch_merge_kernel, grid, dim3(512), 0, s, static_cast<const float*>(a.ws_ml),
+                       static_cast<const float*>(a.ws_o), a.out, a.o_sb, a.o_sh, a.runs, a.group, a.hkv,
+                       a.scale_log2, a.seq_lens, a.batch, a.max_seq_len);
+  else if (a.n_splits > 1)
+    hipLaunchKernelGGL(decode_merge_kernel, grid, dim3(512), 0, s, static_cast<const float*>(a.ws_ml),
+                       static_cast<const float*>(a.ws_o), a.out, a.o_sb, a.o_sh, a.n_splits, a.group, a.hkv,
+                       a.scale_log2);
+  else
+    return hipSuccess;
   return hipGetLastError();
 }
 
