@@ -129,27 +129,34 @@ size_t partial_bytes(int batch, int hkv, int ns) {
   return static_cast<size_t>(batch) * hkv * ns * atf::kDecMaxGroup * (atf::kD + 2) * sizeof(float);
 }
 
-// Runs per kv head of a batch split evenly (decode_batch_kernel), 0 where the
-// splits of decode_split are used.  The lengths are not known here; a batch of
-// equal lengths that decode_split fits to the chip gains nothing by the runs and
-// pays two extra round trips and a few more partials (2 us a call: 6% of 8 x 8K
-// tokens at 8 kv heads, 2.6% of 16 x 8K, 0.3% of 8 x 32K), where a ragged one
-// gains 1.1 to 2 times.  So, by the batch's pages if every sequence were as long
-// as the longest: from 96K pages (768 MB of K and V) on; from 48K on where
-// decode_split's workgroups overfill the chip (12 x 8K tokens: 288 workgroups
-// over 256 CUs, 77 us against 63; 40 x 8K: 320, 215 against 182).  Not for one
-// sequence, nor from 512 sequence x kv head pairs on (two workgroups a CU and no
-// merge: 64 x 8K at 8 kv heads 276 us against 291).
-int batch_runs(int batch, int hkv, int max_seq_len) {
+// Bytes of a spread batch's wave partials.
+size_t spread_bytes(int batch, int hkv, int n_splits, int group) {
+  return static_cast<size_t>(batch) * hkv * n_splits * atf::kDecWaves * group * (atf::kD + 2) * sizeof(float);
+}
+
+// Whether a batch is spread over the chip wave by wave (decode_wave_kernel).  The
+// lengths are not known here, and the results are the same, so the line is one of
+// time, by the batch's pages if every sequence were as long as the longest; us a
+// call against the splits (vec8 k = 2).  The wave partials and their merge cost
+// about 5 us and their bytes, written and read; a ragged batch gains 1.1 to 1.5
+// times, an equal one where its splits overfill the chip (3 x 33000 tokens at 24 / 8
+// heads, 264 workgroups: 74.6 -> 57.3), otherwise little (8 x 12288 57.1 -> 51.6, 32
+// x 3080 61.2 -> 60.0, 32 x 6160 at 28 / 4 heads 58.7 -> 62.0).  From 48K pages on (400
+// MB of K and V), so that those 5 us are at most a tenth.  Fewer than 24 (sequence,
+// kv head) pairs have 11 splits and more each to merge: 2 x 65536 at 28 / 4 heads (8
+// pairs) 34.3 -> 48.7, 4 x 65536 (16 pairs) 64.6 -> 71.5 equal and 46.5 -> 38.3
+// ragged; at twice the pages 16 pairs are worth it (4 x 131072 OFF 166 -> 175 and 93 ->
+// 65), 8 are not (2 x 262144 106 -> 136 and 85 -> 73).  Groups of many heads have
+// partials to match: not where they are more than 1/32 of the pages' bytes (200 x
+// 4096 at 16 / 1 heads, 1/15: 67.7 -> 77.9 equal, 38.5 -> 39.5 ragged; 12 x 65536 at 32
+// / 2, 1/44: 139.5 -> 120.7 and 63.6 -> 55.4).  From 512 pairs on there are two
+// workgroups a CU and nothing to merge.
+bool spread_batch(int batch, int hkv, int n_splits, int waves, int group, int max_seq_len) {
   const int64_t pairs = static_cast<int64_t>(batch) * hkv;
   const int64_t pages = pairs * ((static_cast<int64_t>(max_seq_len) + atf::kPage - 1) / atf::kPage);
-  if (batch <= 1 || pairs >= 512) return 0;
-  const bool overfull = (256 + pairs - 1) / pairs * pairs * 20 > 256 * 21;  // 5% past 256 workgroups
-  if (pages < (overfull ? 48 : 96) * 1024) return 0;
-  return std::max(1, atf::kDecBatchWgs / hkv);
-}
-size_t batch_bytes(int hkv, int runs) {
-  return static_cast<size_t>(hkv) * runs * 2 * atf::kDecMaxGroup * (atf::kD + 2) * sizeof(float);
+  if (batch <= 1 || pairs < 16 || pairs >= 512 || waves != atf::kDecWaves) return false;
+  if (pages < (pairs < 24 ? 96 : 48) * 1024) return false;
+  return spread_bytes(batch, hkv, n_splits, group) * 32 <= static_cast<size_t>(pages) * (atf::kKvBlockElems * 2);
 }
 
 }  // namespace
@@ -260,9 +267,12 @@ size_t atf_decode_workspace_bytes(int batch, int num_q_heads, int num_kv_heads, 
 
 size_t atf_decode_workspace_bytes_even(int batch, int num_q_heads, int num_kv_heads, int max_seq_len) {
   const size_t need = atf_decode_workspace_bytes(batch, num_q_heads, num_kv_heads, max_seq_len);
-  if (batch <= 0 || num_kv_heads <= 0 || max_seq_len <= 0) return need;
-  const int runs = batch_runs(batch, num_kv_heads, max_seq_len);
-  return runs == 0 ? need : std::max(need, batch_bytes(num_kv_heads, runs));
+  if (batch <= 0 || num_kv_heads <= 0 || max_seq_len <= 0 || num_q_heads <= 0 || num_q_heads % num_kv_heads) return need;
+  int ns = 1, pps = 1, waves = 0;
+  decode_split(batch, num_kv_heads, max_seq_len, &ns, &pps, &waves);
+  const int group = num_q_heads / num_kv_heads;
+  if (!spread_batch(batch, num_kv_heads, ns, waves, group, max_seq_len)) return need;
+  return std::max(need, spread_bytes(batch, num_kv_heads, ns, group));
 }
 
 }  // extern "C"
@@ -336,14 +346,17 @@ int decode_prepare(void* out, int64_t o_sb, int64_t o_sh, const void* q, int64_t
                               slice_table, sm_scale, rope_cs, rope_max_pos, layout, a);
 }
 
-// The paged decode's workspace: a batch is split evenly if it holds that split's partials.
-int set_batch_workspace(void* workspace, size_t workspace_bytes, atf::DecodeArgs* a) {
-  const int runs = batch_runs(a->batch, a->hkv, a->max_seq_len);
-  if (runs == 0 || !workspace || !aligned(workspace, 16) || workspace_bytes < batch_bytes(a->hkv, runs)) return 0;
-  a->runs = runs;
-  a->ws_ml = static_cast<float*>(workspace);
-  a->ws_o = a->ws_ml + static_cast<size_t>(a->hkv) * runs * 2 * atf::kDecMaxGroup * 2;
-  return runs;
+// The paged decode's workspace: a batch is spread over the chip if it holds the wave partials.
+bool set_spread_workspace(void* workspace, size_t workspace_bytes, atf::DecodeArgs* a) {
+  if (!spread_batch(a->batch, a->hkv, a->n_splits, a->waves, a->group, a->max_seq_len) || !workspace ||
+      !aligned(workspace, 16) || workspace_bytes < spread_bytes(a->batch, a->hkv, a->n_splits, a->group))
+    return false;
+  const int64_t units = static_cast<int64_t>(a->batch) * a->hkv * a->n_splits * atf::kDecWaves;
+  a->spread = true;
+  a->by_length = units > atf::kDecChipWaves;
+  a->ws_o = static_cast<float*>(workspace);
+  a->ws_ml = a->ws_o + units * a->group * atf::kD;
+  return true;
 }
 
 // The caller's workspace -> the split partials' addresses.
@@ -375,7 +388,7 @@ int decode_with_workspace(void* out, int64_t o_sb, int64_t o_sh, const void* q, 
                              seq_lens, batch, num_q_heads, num_kv_heads, max_seq_len, zhi, slice_table, sm_scale,
                              rope_cs, rope_max_pos, layout, &a))
     return r;
-  if (!set_batch_workspace(workspace, workspace_bytes, &a))
+  if (!set_spread_workspace(workspace, workspace_bytes, &a))
     if (int r = set_workspace(workspace, workspace_bytes, &a)) return r;
   hipError_t e = atf::launch_decode(a, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "decode launch");

@@ -6,11 +6,14 @@
 // kernels/flashinfer_port/fiwin_common.py:96-112, e2e_pipeline/atflash_e2e_fafi.py:106-109;
 // window predicate: kernels/flashinfer_port/decode.cuh.diff:47-89).
 //
-// One workgroup of 8 waves per (sequence, kv head, split of pages); each wave
-// streams its own pages.  The G = Hq/Hkv query heads of the kv head are the 16
-// columns of v_mfma_f32_16x16x32_bf16 (S^T = K Q^T, four 8-dim slices per
-// instruction) and v_mfma_f32_16x16x16_bf16 (O^T = V^T P^T, 16 tokens per
-// instruction).  K and V are loaded straight into the MFMA operand registers.
+// decode_kernel: one workgroup of 8 waves per (sequence, kv head, split of pages);
+// each wave streams its own pages.  decode_wave_kernel: a workgroup per wave, for
+// large batches.  decode_rows_kernel: the same decode over contiguous K and V rows
+// in place of pages.  All three give the same bits.
+//
+// The G = Hq/Hkv query heads of the kv head are the 16 columns of
+// v_mfma_f32_16x16x32_bf16 (S^T = K Q^T, four 8-dim slices per instruction) and
+// v_mfma_f32_16x16x16_bf16 (O^T = V^T P^T, 16 tokens per instruction).  K and V are loaded straight into the MFMA operand registers.
 // The window table is per 8-dim slice (16 entries; a 16-dim level table is
 // passed as each level's value for its two slices).  Page p is read for the
 // first n(p) = #{s : zhi8[s] >= (N-1) - (16p+15)} slices, those its youngest
@@ -26,9 +29,11 @@
 // one split per (sequence, kv head) the workgroup writes the output itself.
 // Otherwise it stores the split's partial in the workspace and ends, and a
 // second kernel (decode_merge_kernel, eight workgroups per (sequence, kv head))
-// merges the split partials by log-sum-exp and writes the output.  The kernel
-// boundary orders the partial stores before the merge loads, so no workgroup
-// waits on another inside a launch: no arrival counters, atomics or fences.
+// merges the split partials by log-sum-exp and writes the output.
+// (decode_wave_kernel stores wave partials, which its merge kernels combine into
+// the split's first.)  The kernel boundary orders the partial stores before the
+// merge loads, so no workgroup waits on another inside a launch: no arrival
+// counters, atomics or fences.
 // (Measured against merging in the last-arriving workgroup of one launch: the
 // chain store -> wait -> arrival atomic -> acquire -> loads there kept a single
 // workgroup busy for about 7 us after the last split finished.)
@@ -191,33 +196,51 @@ __device__ __forceinline__ void dec_load_page(const DecHot& a, int h, int raw, b
   dec_load_v(a, ref, lane, r.v);
 }
 
-// A split's wave partials (m, l, o), in LDS, combined by log-sum-exp: the output
-// where the split is the whole sequence, otherwise the split's partial for
-// decode_merge_kernel.  Thread t owns query heads t / 32 + 2 kWaves j, dims
-// 4 (t % 32) .. +3.
-// part: the partial's index in the workspace; whole: the split is the sequence.
-template <int kWaves>
-__device__ __forceinline__ void store_split(const DecodeArgs& a, int64_t part, bool whole, int h, int b,
-                                            const float* sh_o, const float* sh_m, const float* sh_l) {
+// A split's wave partials (m, l, o) combined by log-sum-exp, wave 0 first: part(w,
+// m, l, o) yields wave w's.  An empty split gives (-inf, 0, 0).
+template <int kWaves, class Part>
+__device__ __forceinline__ void combine_waves(const Part& part, float c, float& M, float& L, f32x4& acc) {
   const float NEG_INF = -__builtin_huge_valf();
+  float m[kWaves], l[kWaves];
+  f32x4 o[kWaves];
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) part(w, m[w], l[w], o[w]);
+  M = NEG_INF;
+  L = 0.f;
+  acc = f32x4{};
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) M = fmaxf(M, m[w]);
+  if (M != NEG_INF) {
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      const float wt = fast_exp2((m[w] - M) * c);  // empty wave: m = -inf -> 0
+      L += wt * l[w];
+      acc += wt * o[w];
+    }
+  }
+}
+
+// The split's wave partials in LDS combined: the output where the split is the
+// whole sequence, otherwise the split's partial for decode_merge_kernel.  Thread t
+// owns query heads t / 32 + 2 kWaves j, dims 4 (t % 32) .. +3.
+// part: the partial's index in the workspace.
+template <int kWaves>
+__device__ __forceinline__ void store_split(const DecodeArgs& a, int64_t part, int h, int b, const float* sh_o,
+                                            const float* sh_m, const float* sh_l) {
   const float c = a.scale_log2;
   const int tid = threadIdx.x;
   const int d4 = 4 * (tid & 31);
   for (int gq = tid >> 5; gq < a.group; gq += 2 * kWaves) {
-    float M = NEG_INF;
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) M = fmaxf(M, sh_m[w * kDecMaxGroup + gq]);
-    float L = 0.f;
-    f32x4 acc = f32x4{};
-    if (M != NEG_INF) {
-#pragma unroll
-      for (int w = 0; w < kWaves; ++w) {
-        const float wt = fast_exp2((sh_m[w * kDecMaxGroup + gq] - M) * c);  // empty wave: m = -inf -> 0
-        L += wt * sh_l[w * kDecMaxGroup + gq];
-        acc += wt * *reinterpret_cast<const f32x4*>(&sh_o[(w * kDecMaxGroup + gq) * kD + d4]);
-      }
-    }
-    if (whole) {  // write the output
+    float M, L;
+    f32x4 acc;
+    combine_waves<kWaves>(
+        [&](int w, float& m, float& l, f32x4& o) {
+          m = sh_m[w * kDecMaxGroup + gq];
+          l = sh_l[w * kDecMaxGroup + gq];
+          o = *reinterpret_cast<const f32x4*>(&sh_o[(w * kDecMaxGroup + gq) * kD + d4]);
+        },
+        c, M, L, acc);
+    if (a.n_splits == 1) {  // write the output
       const float inv = L > 0.f ? 1.f / L : 0.f;
       uint16_t* out = a.out + static_cast<int64_t>(b) * a.o_sb + static_cast<int64_t>(h * a.group + gq) * a.o_sh + d4;
       u32x2 pk;
@@ -232,9 +255,9 @@ __device__ __forceinline__ void store_split(const DecodeArgs& a, int64_t part, b
   }
 }
 
-// Decode of one split (pages `ord`) of sequence b: this wave's pages, its partial
-// (m, l, o) into LDS.  ent: the page-table entries of the wave's first group;
-// wave: its index in the workgroup.
+// Decode of one split (pages `ord`) of sequence b: this wave's pages (kWaves waves
+// take the split), its partial (m, l, o) to row `wave` of sh_o, sh_m and sh_l.
+// ent: the page-table entries of the wave's first group.
 template <bool kPerKey, int kWaves>
 __device__ __forceinline__ void decode_pages(const DecHot& hot, const DecodeArgs& a, int h, int b, int N,
                                              const int32_t* row, const PageOrder& ord, int wave, int p_first,
@@ -445,169 +468,91 @@ void decode_kernel(const int32_t* page_table, const int32_t* seq_lens, const uin
   set_page_count(ord, s, hot.n_splits, hot.pages_per_split, n_pages);
   decode_pages<kPerKey, kWaves>(hot, a, h, b, N, row, ord, wave, p_first, ent, sh_o, sh_m, sh_l);
   __syncthreads();
-  store_split<kWaves>(a, (static_cast<int64_t>(b) * hot.hkv + h) * a.n_splits + s, a.n_splits == 1, h, b, sh_o, sh_m, sh_l);
+  store_split<kWaves>(a, (static_cast<int64_t>(b) * hot.hkv + h) * a.n_splits + s, h, b, sh_o, sh_m, sh_l);
 }
 
-// ---- a batch split evenly over the chip ----
+// ---- a batch spread over the chip wave by wave ----
 // decode_kernel's grid gives every sequence of a batch the splits of the longest
-// one, as many as fit 256 workgroups: a ragged batch leaves most workgroups with
-// little to do, and sequence x kv head counts that do not divide 256 either leave
-// CUs idle or start a second wave of workgroups (12 sequences x 8 kv heads: 288).
-// Here the pages of the whole batch, one sequence after the other, are cut into
-// `chunks` equal runs per kv head (kDecBatchWgs = 256 workgroups in all, one per
-// CU), and workgroup (c, h) decodes run c: the end of one sequence, whole ones,
-// the beginning of another.  The lengths live in device memory, so every
-// workgroup derives its run from them (one load per 64 sequences, sums by DPP).
-// A sequence inside one run is written by its workgroup; a cut one leaves a
-// partial per run, merged by decode_batch_merge_kernel.  Run c's partials are 2c
-// (of a sequence that it begins with) and 2c + 1 (of one that begins inside it).
-//   HBM bound.  Measured against decode_kernel on the same batch (24 / 8 heads,
-// vec8 k = 2; us a call): 12 sequences of 700 to 32768 tokens 110 -> 73, 16 of
-// them 157 -> 80, 12 of 32K 266 -> 202, 40 of 8K 214 -> 185, 8 of 32K (equal, 256
-// splits either way) 134.6 -> 135.8.  512 workgroups of 4 waves instead: ragged
-// batches the same within 6%, equal ones of 32K 5% slower.
-struct BatchPlan {
-  int run;   // virtual pages per run
-  int gran;  // a sequence takes a multiple of this many virtual pages
-  int nsb;   // > 0: nearly equal lengths; every sequence takes nsb runs, interleaved page by page
-};
+// one, as many as fit 256 workgroups, and a workgroup keeps a split's eight waves
+// on one CU: a ragged batch leaves most CUs with little to do while a few stream
+// the long sequences, and sequence x kv head counts that do not divide 256 start a
+// second wave of workgroups.  Here every wave of every split is a workgroup of its
+// own, so that the waves of a long sequence spread over all CUs; where there are
+// more of them than the chip holds (eight a CU), those of the longest sequences
+// are dispatched first.  The lengths live in device memory: a wave finds the
+// sequence that its place in the grid means from them.
+// Pages, page order and arithmetic of a wave are decode_kernel's, and
+// decode_wave_merge_kernel combines waves and splits in decode_kernel's and
+// decode_merge_kernel's order: the outputs are theirs bit for bit, whatever the
+// other sequences of the batch hold.
+//   HBM bound.  Against decode_kernel and its merge on the same batch (24 / 8
+// heads, vec8 k = 2; us a call): 12 sequences of 700 to 32768 tokens 110.8 -> 69.8,
+// 40 of 300 to 9000 (level table) 99.3 -> 67.3, 12 of 32768 261 -> 207, 40 of 8192
+// 210 -> 177, 8 of 32768 124.5 -> 123.4.  At 168 registers, three waves a SIMD, the
+// page registers spill: 12 ragged sequences 274.
+constexpr int kDecSpreadBatch = 512;  // sequences at most
 
-// Lengths of the 64 sequences from b0 on, one per lane (0 past the batch).
-__device__ __forceinline__ int batch_lens(const int32_t* seq_lens, int batch, int max_seq_len, int b0) {
-  const int b = b0 + static_cast<int>(threadIdx.x & 63);
-  return b < batch ? max(0, min(seq_lens[b], max_seq_len)) : 0;
-}
-__device__ __forceinline__ int len_pages(int n) { return (n + kPage - 1) / kPage; }
-
-// Inclusive prefix sum (or maximum) over the wave's 64 lanes by DPP (VALU moves:
-// row shifts by 1, 2, 4, 8, then the row broadcasts); lane 63 has the total.
-template <class Op>
-__device__ __forceinline__ int wave_scan(int x, const Op& op) {
-  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, true));
-  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, true));
-  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, true));
-  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, true));
-  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false));
-  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false));
-  return x;
-}
-__device__ __forceinline__ int scan_sum(int x) {
-  return wave_scan(x, [](int a, int b) { return a + b; });
-}
-
-// The runs of a batch; every wave computes the same plan.  lens0: batch_lens of
-// the first 64 sequences.
-//   Short batches (each sequence's pages by the 32 fit the runs): runs of 32
-// pages, one 4-page group per wave, no run across two sequences.
-//   Nearly equal lengths (the longest within 4% of the mean) that divide the
-// runs (5% left over at most): each sequence in nsb splits of its own,
-// interleaved page by page as decode_kernel's are.
-//   Otherwise equal runs, in groups of 4 pages.
-__device__ __forceinline__ BatchPlan batch_plan(const int32_t* seq_lens, int batch, int max_seq_len, int chunks,
-                                                int lens0) {
-  constexpr int kRun = kDecUnroll * kDecBatchWaves;  // one 4-page group per wave
-  int t4 = 0, tr = 0, mx = 0;
-  for (int b0 = 0; b0 < batch; b0 += 64) {
-    const int p = len_pages(b0 == 0 ? lens0 : batch_lens(seq_lens, batch, max_seq_len, b0));
-    t4 += __builtin_amdgcn_readlane(scan_sum((p + 3) & ~3), 63);
-    tr += __builtin_amdgcn_readlane(scan_sum((p + kRun - 1) / kRun), 63);
-    mx = max(mx, __builtin_amdgcn_readlane(wave_scan(p, [](int a, int b) { return max(a, b); }), 63));
-  }
-  if (tr <= chunks) return BatchPlan{kRun, kRun, 0};
-  const int nsb = chunks / batch;
-  if (nsb > 0 && static_cast<int64_t>(mx) * batch * 100 <= static_cast<int64_t>(t4) * 104 &&
-      nsb * batch * 20 >= chunks * 19)
-    return BatchPlan{0, 0, nsb};
-  return BatchPlan{((t4 + chunks - 1) / chunks + 3) & ~3, 4, 0};
-}
-
-// The first sequence that ends past virtual page `at` (find) or sequence `at`,
-// the virtual page x it starts at, and its 64 sequences' lengths (lens; lens0 on
-// entry).  b = batch if there is none.
-__device__ __forceinline__ void batch_locate(const int32_t* seq_lens, int batch, int max_seq_len, int gran, bool find,
-                                             int at, int& lens, int& b, int& x) {
+// The sequence of rank r by length in pages (0: the longest; equal lengths by
+// index).  r < batch <= 64 kRegs; every lane of the wave takes part.
+template <int kRegs>
+__device__ __forceinline__ int nth_longest(const int32_t* seq_lens, int batch, int max_seq_len, int r) {
   const int lane = threadIdx.x & 63;
-  int base = 0;
-  for (int b0 = 0; b0 < batch; b0 += 64) {
-    if (b0 > 0) lens = batch_lens(seq_lens, batch, max_seq_len, b0);
-    const int v = (len_pages(lens) + gran - 1) & ~(gran - 1);
-    const int incl = scan_sum(v);
-    const uint64_t hit = __builtin_amdgcn_ballot_w64(find ? base + incl > at : b0 + lane == at);
-    if (hit != 0) {
-      const int l = __builtin_ctzll(hit);
-      b = b0 + l;
-      x = base + __builtin_amdgcn_readlane(incl - v, l);
-      return;
-    }
-    base += __builtin_amdgcn_readlane(incl, 63);
+  int p[kRegs];  // pages of sequence 64 i + lane (-1 past the batch)
+#pragma unroll
+  for (int i = 0; i < kRegs; ++i) {
+    const int b = 64 * i + lane;
+    p[i] = b < batch ? (max(0, min(seq_lens[b], max_seq_len)) + kPage - 1) / kPage : -1;
   }
-  b = batch;
-  x = base;
+  auto count = [&](int at_least) {
+    int n = 0;
+#pragma unroll
+    for (int i = 0; i < kRegs; ++i) n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(p[i] >= at_least));
+    return n;
+  };
+  int t = 0;  // the largest page count that more than r sequences reach
+  for (int bit = 1 << (31 - __builtin_clz(max_seq_len / kPage + 1)); bit != 0; bit >>= 1)
+    if (count(t | bit) > r) t |= bit;
+  int k = r - count(t + 1);  // the k-th of the sequences of t pages
+  int found = 0;
+#pragma unroll
+  for (int i = 0; i < kRegs; ++i) {
+    const uint64_t eq = __builtin_amdgcn_ballot_w64(p[i] == t);
+    const int below = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(eq >> 32),
+                                                __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(eq), 0u));
+    const uint64_t hit = __builtin_amdgcn_ballot_w64(p[i] == t && below == k);
+    if (hit != 0) found = 64 * i + __builtin_ctzll(hit);
+    k -= __builtin_popcountll(eq);
+  }
+  return found;
 }
 
+// grid: x = split, y = kv head + kv heads x wave, z = the sequence, or its rank by
+// length (a.by_length).  Pages that lie side by side, and a page's blocks of the kv
+// heads, are then read at about the same time: with the waves of a split before
+// the heads 32 x 16K tokens take 280 us and not 261 (24 / 8 heads, vec8 k = 2), with
+// heads and waves before the splits 4 x 128K 196 and not 176 (28 / 4 heads, OFF).
 template <bool kPerKey>
-__global__ __launch_bounds__(kDecBatchWaves * 64) __attribute__((amdgpu_waves_per_eu(2)))
-void decode_batch_kernel(const int32_t* page_table, const int32_t* seq_lens, const uint16_t* kv_cache, int max_pages,
-                         int chunks, int max_seq_len, int hkv, int num_pages, int batch, DecodeArgs a) {
-  constexpr int kWaves = kDecBatchWaves;
-  const DecHot hot{page_table, seq_lens, kv_cache, max_pages, 0, max_seq_len, hkv, num_pages, 1};
-  __shared__ __attribute__((aligned(16))) float sh_o[kWaves * kDecMaxGroup * kD];
-  __shared__ float sh_m[kWaves * kDecMaxGroup], sh_l[kWaves * kDecMaxGroup];
-  const int c = blockIdx.x + gridDim.x * blockIdx.z, h = blockIdx.y;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
+void decode_wave_kernel(const int32_t* page_table, const int32_t* seq_lens, const uint16_t* kv_cache, int max_pages,
+                        int pages_per_split, int max_seq_len, int hkv, int num_pages, int n_splits, DecodeArgs a) {
+  const DecHot hot{page_table, seq_lens, kv_cache, max_pages, pages_per_split, max_seq_len, hkv, num_pages, n_splits};
+  const int s = blockIdx.x, h = blockIdx.y % hkv, wave = blockIdx.y / hkv;
+  int b = blockIdx.z;
+  if (a.by_length) b = a.batch <= 64 ? nth_longest<1>(seq_lens, a.batch, max_seq_len, b)
+                                     : nth_longest<kDecSpreadBatch / 64>(seq_lens, a.batch, max_seq_len, b);
   const int p_first = kDecUnroll * wave;
-  int lens = batch_lens(seq_lens, batch, max_seq_len, 0);
-  // The first group's page-table entries if the lengths turn out nearly equal
-  // (this run: split s of sequence bu, interleaved), fetched with the lengths,
-  // their index clamped into the table row: that case then waits for no more
-  // memory round trips than decode_kernel does.
-  const int nsb = chunks / batch;
-  const int bu = nsb > 0 ? min(c / nsb, batch - 1) : 0, su = nsb > 0 ? c - c / nsb * nsb : 0;
+  PageOrder ord = page_order(s, n_splits, pages_per_split);
   int ent[kDecUnroll];
+  const int32_t* row = page_table + static_cast<int64_t>(b) * max_pages;
 #pragma unroll
-  for (int u = 0; u < kDecUnroll; ++u)
-    ent[u] = page_table[static_cast<int64_t>(bu) * max_pages + min(su + max(nsb, 1) * (p_first + u), max_pages - 1)];
-  const BatchPlan bp = batch_plan(seq_lens, batch, max_seq_len, chunks, lens);
-  int b, x = 0;
-  const int begin = c * bp.run, end = begin + bp.run;
-  if (bp.nsb > 0) {
-    b = c / bp.nsb;
-    if (b >= 64) lens = batch_lens(seq_lens, batch, max_seq_len, b & ~63);
-  } else {
-    batch_locate(seq_lens, batch, max_seq_len, bp.gran, true, begin, lens, b, x);
-  }
-  bool first = true;
-  while (b < batch && (bp.nsb > 0 ? first : x < end)) {
-    const int N = __builtin_amdgcn_readlane(lens, b & 63);
-    const int P = len_pages(N);
-    PageOrder ord;
-    bool whole;
-    if (bp.nsb > 0) {
-      const int s = c - b * bp.nsb;
-      ord = PageOrder{s, bp.nsb, P > s ? (P - s + bp.nsb - 1) / bp.nsb : 0};
-      whole = bp.nsb == 1;
-    } else {
-      const int p0 = max(begin - x, 0), p1 = min(end - x, P);
-      ord = PageOrder{p0, 1, max(p1 - p0, 0)};
-      whole = p0 == 0 && p1 == P;
-    }
-    if (ord.count > 0 || bp.nsb > 0) {
-      if (!first) __syncthreads();  // the last sequence's partials in LDS have been read
-      const int32_t* row = page_table + static_cast<int64_t>(b) * max_pages;
-      if (bp.nsb == 0) {
-#pragma unroll
-        for (int u = 0; u < kDecUnroll; ++u) ent[u] = dec_fetch_entry(row, ord, p_first + u);
-      }
-      decode_pages<kPerKey, kWaves>(hot, a, h, b, N, row, ord, wave, p_first, ent, sh_o, sh_m, sh_l);
-      __syncthreads();
-      const int64_t part = static_cast<int64_t>(h) * 2 * chunks + 2 * c + (bp.nsb == 0 && x > begin ? 1 : 0);
-      store_split<kWaves>(a, part, whole, h, b, sh_o, sh_m, sh_l);
-      first = false;
-    }
-    if (bp.nsb > 0) break;
-    x += (P + bp.gran - 1) & ~(bp.gran - 1);
-    if ((++b & 63) == 0) lens = batch_lens(seq_lens, batch, max_seq_len, b);
-  }
+  for (int u = 0; u < kDecUnroll; ++u) ent[u] = row[min(ord.po + ord.pm * (p_first + u), max_pages - 1)];
+  const int N = max(0, min(seq_lens[b], max_seq_len));
+  set_page_count(ord, s, n_splits, pages_per_split, (N + kPage - 1) / kPage);
+  // wave partials: o [(sequence, kv head, split, wave)][group][128], then m [group] and l [group] of each
+  const int64_t unit = ((static_cast<int64_t>(b) * hkv + h) * n_splits + s) * kDecWaves + wave;
+  float* ml = a.ws_ml + unit * 2 * a.group;
+  decode_pages<kPerKey, kDecWaves>(hot, a, h, b, N, row, ord, 0, p_first, ent, a.ws_o + unit * a.group * kD, ml,
+                                   ml + a.group);
 }
 
 // ---- decode over contiguous K and V rows ----
@@ -838,7 +783,7 @@ void decode_rows_kernel(RowsArgs ra) {
     }
   }
   __syncthreads();
-  store_split<kWaves>(a, (static_cast<int64_t>(b) * a.hkv + h) * a.n_splits + s, a.n_splits == 1, h, b, sh_o, sh_m, sh_l);
+  store_split<kWaves>(a, (static_cast<int64_t>(b) * a.hkv + h) * a.n_splits + s, h, b, sh_o, sh_m, sh_l);
 }
 
 // ---- measurement probe: the streaming ceiling of the decode's page loads ----
@@ -966,7 +911,8 @@ __device__ __forceinline__ float row_ror(float x) {
 // the lane one row (two rows) away: afterwards every lane of a group {4h + q}
 // holds the merge of the group's partials.  Every lane takes part; the caller
 // keeps control flow uniform around it.
-__device__ __forceinline__ void merge_lane_groups(float& m, float& l, f32x4& o, bool whole_wave, float c) {
+// merge_rows: the row rotations alone, for groups that lie in a 16-lane row.
+__device__ __forceinline__ void merge_rows(float& m, float& l, f32x4& o, float c) {
   {
     f32x4 op;
 #pragma unroll
@@ -979,6 +925,9 @@ __device__ __forceinline__ void merge_lane_groups(float& m, float& l, f32x4& o, 
     for (int i = 0; i < 4; ++i) op[i] = row_ror<4>(o[i]);
     merge_pair(m, l, o, row_ror<4>(m), row_ror<4>(l), op, c);
   }
+}
+__device__ __forceinline__ void merge_lane_groups(float& m, float& l, f32x4& o, bool whole_wave, float c) {
+  merge_rows(m, l, o, c);
   // a swap of a register with itself: result [0] holds rows (0, 0, 2, 2) and
   // result [1] rows (1, 1, 3, 3) of the value (32-lane swap: halves (0, 0) and
   // (1, 1)), so merging [0] with [1] merges each lane with its partner lane
@@ -1018,14 +967,36 @@ __device__ __forceinline__ void merge_lane_groups(float& m, float& l, f32x4& o, 
   }
 }
 
-// kBatch: the partials of decode_batch_kernel (n_splits holds the runs per kv
-// head); a sequence in one run has its output already, an empty one is zeroed here.
-template <bool kBatch>
-__device__ __forceinline__ void merge_splits(MergeArgs a, const int32_t* seq_lens, int batch, int max_seq_len) {
-  const int n_splits = a.n_splits;
+// The output row of query head hq_idx, dims md4 .. +3.
+__device__ __forceinline__ void store_merged(const MergeArgs& a, int b, int hq_idx, int md4, float l, const f32x4& o) {
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  uint16_t* out = a.out + static_cast<int64_t>(b) * a.o_sb + static_cast<int64_t>(hq_idx) * a.o_sh + md4;
+  u32x2 pk;
+  pk[0] = pack_bf16x2(o[0] * inv, o[1] * inv);
+  pk[1] = pack_bf16x2(o[2] * inv, o[3] * inv);
+  *reinterpret_cast<u32x2*>(out) = pk;
+}
+
+// The wave partials of a split (decode_wave_kernel's; split: its index in the call)
+// combined, for query head mg of the group and dims md4 .. +3.
+__device__ __forceinline__ void load_wave_split(const MergeArgs& a, int64_t split, int mg, int md4, float& M, float& L,
+                                                f32x4& acc) {
+  combine_waves<kDecWaves>(
+      [&](int w, float& m, float& l, f32x4& o) {
+        const int64_t u = split * kDecWaves + w;
+        const float* ml = a.ws_ml + u * 2 * a.group + mg;
+        m = ml[0];
+        l = ml[a.group];
+        o = *reinterpret_cast<const f32x4*>(a.ws_o + (u * a.group + mg) * kD + md4);
+      },
+      a.scale_log2, M, L, acc);
+}
+
+// kWavePartials: the partials are decode_wave_kernel's, a split's combined as it is loaded.
+template <bool kWavePartials>
+__device__ __forceinline__ void merge_splits(const MergeArgs& a) {
   const int chunk = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-  int64_t part0 = (static_cast<int64_t>(b) * a.hkv + h) * a.n_splits;  // split 0's partial
-  int step = 1, skew = 0;  // split i's is part0 + step * i, less skew after the first
+  const int64_t part0 = (static_cast<int64_t>(b) * a.hkv + h) * a.n_splits;  // split 0's partial
   const int tid = threadIdx.x;
   const float NEG_INF = -__builtin_huge_valf();
   const float c = a.scale_log2;
@@ -1035,49 +1006,29 @@ __device__ __forceinline__ void merge_splits(MergeArgs a, const int32_t* seq_len
   const int q4 = 4 * (tid % kMergeLanes);
   const int md4 = chunk * kMergeDims + q4;
   const bool mact = mg < a.group;
-  f32x2 mlv[kMergeBatch];
-  f32x4 ov[kMergeBatch];
-  auto load = [&](int j0) {
-#pragma unroll
-    for (int j = 0; j < kMergeBatch; ++j) {
-      const int sp = j0 + j * H;
-      mlv[j] = f32x2{NEG_INF, 0.f};
-      ov[j] = f32x4{};
-      if (mact && sp < a.n_splits) {
-        const int64_t pi = (part0 + step * sp - (sp > 0 ? skew : 0)) * kDecMaxGroup + mg;
-        mlv[j] = *reinterpret_cast<const f32x2*>(a.ws_ml + pi * 2);
-        ov[j] = *reinterpret_cast<const f32x4*>(a.ws_o + pi * kD + md4);
-      }
-    }
-  };
-  if constexpr (kBatch) {
-    // The partials of the nearly-equal-lengths layout are loaded along with the
-    // lengths that decide whether it is the one (if not, they are not used).
-    int lens = batch_lens(seq_lens, batch, max_seq_len, 0);
-    const int nsb = n_splits / batch;
-    part0 = static_cast<int64_t>(h) * 2 * n_splits + 2 * b * nsb;
-    step = 2;
-    a.n_splits = nsb;
-    load(hh);
-    const BatchPlan bp = batch_plan(seq_lens, batch, max_seq_len, n_splits, lens);
-    if (bp.nsb == 0) {
-      int bb = b, x = 0;
-      batch_locate(seq_lens, batch, max_seq_len, bp.gran, false, b, lens, bb, x);
-      const int c0 = x / bp.run, P = len_pages(__builtin_amdgcn_readlane(lens, b & 63));
-      a.n_splits = P > 0 ? (x + P - 1) / bp.run - c0 + 1 : 0;
-      skew = x > c0 * bp.run ? 1 : 0;
-      part0 = static_cast<int64_t>(h) * 2 * n_splits + 2 * c0 + skew;
-    }
-    if (a.n_splits == 1) return;
-    if (bp.nsb == 0) load(hh);
-  } else {
-    load(hh);
-  }
   float m_t = NEG_INF, L_t = 0.f;
   f32x4 acc_t = f32x4{};
   if (mact) {
     for (int j0 = hh; j0 < a.n_splits; j0 += kMergeBatch * H) {
-      if (j0 != hh) load(j0);
+      f32x2 mlv[kMergeBatch];
+      f32x4 ov[kMergeBatch];
+#pragma unroll
+      for (int j = 0; j < kMergeBatch; ++j) {
+        const int sp = j0 + j * H;
+        mlv[j] = f32x2{NEG_INF, 0.f};
+        ov[j] = f32x4{};
+        if (sp < a.n_splits) {
+          if constexpr (kWavePartials) {
+            float M, L;
+            load_wave_split(a, part0 + sp, mg, md4, M, L, ov[j]);
+            mlv[j] = f32x2{M, L};
+          } else {
+            const int64_t pi = (part0 + sp) * kDecMaxGroup + mg;
+            mlv[j] = *reinterpret_cast<const f32x2*>(a.ws_ml + pi * 2);
+            ov[j] = *reinterpret_cast<const f32x4*>(a.ws_o + pi * kD + md4);
+          }
+        }
+      }
       float mb = m_t;
 #pragma unroll
       for (int j = 0; j < kMergeBatch; ++j) mb = fmaxf(mb, mlv[j][0]);
@@ -1099,32 +1050,43 @@ __device__ __forceinline__ void merge_splits(MergeArgs a, const int32_t* seq_len
   // empty partial); lanes 4k + (t % 4), k < H, hold one (head, dims): 16
   // groups per wave for G <= 8, 8 per half wave above
   merge_lane_groups(m_t, L_t, acc_t, H == 16, c);
-  if (mact && hh == 0) {
-    const float inv = L_t > 0.f ? 1.f / L_t : 0.f;
-    uint16_t* out = a.out + static_cast<int64_t>(b) * a.o_sb + static_cast<int64_t>(h * a.group + mg) * a.o_sh + md4;
-    u32x2 pk;
-    pk[0] = pack_bf16x2(acc_t[0] * inv, acc_t[1] * inv);
-    pk[1] = pack_bf16x2(acc_t[2] * inv, acc_t[3] * inv);
-    *reinterpret_cast<u32x2*>(out) = pk;
-  }
+  if (mact && hh == 0) store_merged(a, b, h * a.group + mg, md4, L_t, acc_t);
 }
 
-// The lengths are the batch kernel's own arguments: 56 bytes of arguments are one
-// line to write per launch, 72 are two, on a path where the host sets the time
-// (8K tokens, one sequence: 13.0 -> 11.5 to 12.0 us a call; 1003 by a plan: 10.3 ->
-// 9.1 to 10.1).
 __global__ __launch_bounds__(512) void decode_merge_kernel(const float* ws_ml, const float* ws_o, uint16_t* out,
                                                            int64_t o_sb, int64_t o_sh, int n_splits, int group,
                                                            int hkv, float scale_log2) {
-  merge_splits<false>(MergeArgs{ws_ml, ws_o, out, o_sb, o_sh, n_splits, group, hkv, scale_log2}, nullptr, 0, 0);
+  merge_splits<false>(MergeArgs{ws_ml, ws_o, out, o_sb, o_sh, n_splits, group, hkv, scale_log2});
 }
 
-__global__ __launch_bounds__(512) void decode_batch_merge_kernel(const float* ws_ml, const float* ws_o, uint16_t* out,
-                                                                 int64_t o_sb, int64_t o_sh, int n_splits, int group,
-                                                                 int hkv, float scale_log2, const int32_t* seq_lens,
-                                                                 int batch, int max_seq_len) {
-  merge_splits<true>(MergeArgs{ws_ml, ws_o, out, o_sb, o_sh, n_splits, group, hkv, scale_log2}, seq_lens, batch,
-                     max_seq_len);
+// The merge after decode_wave_kernel: eight wave partials a split, then the splits.
+__global__ __launch_bounds__(512) void decode_wave_merge_kernel(const float* ws_ml, const float* ws_o, uint16_t* out,
+                                                                int64_t o_sb, int64_t o_sh, int n_splits, int group,
+                                                                int hkv, float scale_log2) {
+  merge_splits<true>(MergeArgs{ws_ml, ws_o, out, o_sb, o_sh, n_splits, group, hkv, scale_log2});
+}
+
+// The same for at most kSplits (1 or 4) splits, without idle lanes for the splits
+// and heads that are not there: 4 kSplits lanes take 16 dims of a query head, the
+// rows (sequence, query head, 16 dims) lie one after the other.  The sums are
+// merge_splits', whose further exchanges meet empty partials here.
+constexpr int kMergeFewThreads = 256;
+template <int kSplits>
+__global__ __launch_bounds__(kMergeFewThreads) void decode_wave_merge_few_kernel(
+    const float* ws_ml, const float* ws_o, uint16_t* out, int64_t o_sb, int64_t o_sh, int n_splits, int group, int hkv,
+    float scale_log2, int rows) {
+  static_assert(kSplits == 1 || kSplits == 4, "one lane group, or the four of a 16-lane row");
+  const MergeArgs a{ws_ml, ws_o, out, o_sb, o_sh, n_splits, group, hkv, scale_log2};
+  const int t = blockIdx.x * kMergeFewThreads + threadIdx.x;
+  const int row = t / (kMergeLanes * kSplits), sp = t / kMergeLanes % kSplits;
+  const int md4 = row % kMergeChunks * kMergeDims + 4 * (t % kMergeLanes);
+  const int head = row / kMergeChunks;                 // sequence, query head
+  const int pair = head / group, mg = head % group;    // sequence, kv head
+  float M = -__builtin_huge_valf(), L = 0.f;
+  f32x4 acc = f32x4{};
+  if (row < rows && sp < n_splits) load_wave_split(a, static_cast<int64_t>(pair) * n_splits + sp, mg, md4, M, L, acc);
+  if constexpr (kSplits > 1) merge_rows(M, L, acc, scale_log2);
+  if (row < rows && sp == 0) store_merged(a, pair / hkv, pair % hkv * group + mg, md4, L, acc);
 }
 
 // Level count per page for one sequence of length N under the page rule
@@ -1136,38 +1098,32 @@ __global__ void decode_page_levels_kernel(int32_t* out, int n_pages, int N, Leve
   out[p] = levels_of(lt, max(0, (N - 1) - (p * kPage + kPage - 1)));
 }
 
-// The merge of a call's split partials (nothing to do with one split).
+// The merge of a call's split partials (nothing to do with one split in one workgroup).
 static hipError_t launch_merge(const DecodeArgs& a, hipStream_t s) {
-  const dim3 grid(kMergeChunks, a.hkv, a.batch);
-  if (a.runs > 0)
-    hipLaunchKernelGGL(decode_batch_merge_kernel, grid, dim3(512), 0, s, static_cast<const float*>(a.ws_ml),
-                       static_cast<const float*>(a.ws_o), a.out, a.o_sb, a.o_sh, a.runs, a.group, a.hkv,
-                       a.scale_log2, a.seq_lens, a.batch, a.max_seq_len);
-  else if (a.n_splits > 1)
-    hipLaunchKernelGGL(decode_merge_kernel, grid, dim3(512), 0, s, static_cast<const float*>(a.ws_ml),
-                       static_cast<const float*>(a.ws_o), a.out, a.o_sb, a.o_sh, a.n_splits, a.group, a.hkv,
-                       a.scale_log2);
-  else
-    return hipSuccess;
+  if (!a.spread && a.n_splits == 1) return hipSuccess;
+  const float *ml = a.ws_ml, *o = a.ws_o;
+  if (a.spread && a.n_splits <= 4) {
+    const int rows = a.batch * a.hq * kMergeChunks, lanes = kMergeLanes * (a.n_splits == 1 ? 1 : 4);
+    const dim3 grid((rows * lanes + kMergeFewThreads - 1) / kMergeFewThreads);
+    hipLaunchKernelGGL(a.n_splits == 1 ? decode_wave_merge_few_kernel<1> : decode_wave_merge_few_kernel<4>, grid,
+                       dim3(kMergeFewThreads), 0, s, ml, o, a.out, a.o_sb, a.o_sh, a.n_splits, a.group, a.hkv,
+                       a.scale_log2, rows);
+  } else {
+    hipLaunchKernelGGL(a.spread ? decode_wave_merge_kernel : decode_merge_kernel, dim3(kMergeChunks, a.hkv, a.batch),
+                       dim3(512), 0, s, ml, o, a.out, a.o_sb, a.o_sh, a.n_splits, a.group, a.hkv, a.scale_log2);
+  }
   return hipGetLastError();
 }
 
 hipError_t launch_decode(const DecodeArgs& a, hipStream_t s) {
   if (a.batch <= 0) return hipSuccess;
-  if (a.runs > 0) {
-    // Block order: the runs of a sequence, then the kv heads, then the sequences,
-    // as decode_kernel's, where equal lengths give a sequence four runs or more
-    // (16 sequences of 32K, 4 kv heads: 138 us; all runs of a head side by side:
-    // 145) and no run is left over (its empty workgroups would upset the even
-    // spread over the CUs: 5 sequences of 32K, 8 kv heads: 130 us against 115);
-    // otherwise the latter (64 of 8K, 4 kv heads: 149 against 157).
-    const int nsb = a.runs / a.batch, side = nsb >= 4 && nsb * a.batch == a.runs ? nsb : a.runs;
-    const dim3 grid(side, a.hkv, a.runs / side);
-#define ATF_BATCH_LAUNCH(PK)                                                                                        \
-  hipLaunchKernelGGL(decode_batch_kernel<PK>, grid, dim3(kDecBatchWaves * 64), 0, s, a.page_table, a.seq_lens,     \
-                     a.kv_cache, a.max_pages, a.runs, a.max_seq_len, a.hkv, a.num_pages, a.batch, a)
-    if (a.per_key) ATF_BATCH_LAUNCH(true); else ATF_BATCH_LAUNCH(false);
-#undef ATF_BATCH_LAUNCH
+  if (a.spread) {
+#define ATF_WAVE_LAUNCH(PK)                                                                                        \
+  hipLaunchKernelGGL(decode_wave_kernel<PK>, dim3(a.n_splits, a.hkv * kDecWaves, a.batch), dim3(64), 0, s,          \
+                     a.page_table, a.seq_lens, a.kv_cache, a.max_pages, a.pages_per_split, a.max_seq_len, a.hkv,     \
+                     a.num_pages, a.n_splits, a)
+    if (a.per_key) ATF_WAVE_LAUNCH(true); else ATF_WAVE_LAUNCH(false);
+#undef ATF_WAVE_LAUNCH
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     return launch_merge(a, s);
   }

@@ -20,8 +20,7 @@ constexpr int kDecUnroll = 4;      // pages in flight per wave
 constexpr int kDecWaves = 8;       // waves per workgroup (one split), 2 per SIMD
 constexpr int kDecWavesShort = 4;  // the same for contexts too short to give 256 splits of 8 waves
 constexpr int kDecMaxSplits = 256;
-constexpr int kDecBatchWaves = 8;   // waves per workgroup of a batch split evenly
-constexpr int kDecBatchWgs = 2048 / kDecBatchWaves;  // its workgroups: two waves per SIMD
+constexpr int kDecChipWaves = 2048;  // waves of a decode that the chip holds: two per SIMD
 // Fixed device scratch of the entry point that allocates nothing
 // (atf_decode_paged_bf16_noalloc): split partials, laid out as in a workspace.
 constexpr size_t kDecScratchBytes = size_t(8) << 20;
@@ -74,7 +73,8 @@ struct DecodeArgs {
   int batch, hq, hkv, group;
   int n_splits, pages_per_split;
   int waves;  // kDecWaves or kDecWavesShort per workgroup
-  int runs;   // > 0: the batch in this many equal runs per kv head (decode_batch_kernel)
+  bool spread;     // one workgroup per wave of a split (decode_wave_kernel); waves = kDecWaves
+  bool by_length;  // with spread: the longest sequences' waves first
   float scale_log2;
   const float* rope_cs;
   int layout;
@@ -85,8 +85,9 @@ struct DecodeArgs {
   LevelTable lt;
   SliceTable st;
   int per_key;
-  float* ws_ml;        // [B][Hkv][n_splits][16][2]   split partials (n_splits > 1);
-  float* ws_o;         // [B][Hkv][n_splits][16][128] with runs [Hkv][2 runs][16][2 or 128]
+  // partials: of splits (n_splits > 1), or with spread of the splits' waves
+  float* ws_ml;        // [B][Hkv][n_splits][16][2],   [B][Hkv][n_splits][8][2][group]
+  float* ws_o;         // [B][Hkv][n_splits][16][128], [B][Hkv][n_splits][8][group][128]
 };
 
 // K and V of a contiguous decode: rows [batch][token][head][128] (element strides).

@@ -128,11 +128,12 @@ int atf_prefill_bf16(void* out, int64_t o_sb, int64_t o_st, int64_t o_sh, float*
 size_t atf_decode_workspace_bytes(int batch, int num_q_heads, int num_kv_heads, int max_seq_len);
 
 /*
- * Bytes of device workspace with which the paged decode splits a batch evenly
- * over the chip, whatever the sequences' lengths (at least
- * atf_decode_workspace_bytes; at most about 4.1 MiB).  With less, down to
- * atf_decode_workspace_bytes, every sequence gets the splits of the longest.
- * The two differ in the order of fp32 sums, so in the last bits of the results.
+ * Bytes of device workspace with which the paged decode spreads a batch over the
+ * whole chip whatever its sequences' lengths (at least
+ * atf_decode_workspace_bytes; at most about 34 MB).  With less, down to
+ * atf_decode_workspace_bytes, every sequence gets the splits of the longest on as
+ * many workgroups, which is slower for a ragged batch.  The results are the same
+ * bit for bit.
  */
 size_t atf_decode_workspace_bytes_even(int batch, int num_q_heads, int num_kv_heads, int max_seq_len);
 
