@@ -960,9 +960,17 @@ __device__ __forceinline__ void qk_blocks(uint64_t lm, const lds_u8* kb, const u
 // CUs idle or more there.  Without a partner on its SIMD, a wave overlaps its own
 // work: the softmax of pair u sits between the MFMAs of the PV of pair u-1, which
 // it does not depend on (pv_softmax_stream), then come the rescale check and the
-// QK of pair u+1; one barrier per pair.  The copies are spread over the MFMAs row
-// by row, V of pair u during its PV part, K of pair u+3 during its QK part, and
-// the scalar work (level counts, page addresses) is done between them.  Every
+// QK of pair u+1; one barrier per pair.
+//   The ring (B_u: the barrier that ends iteration u; B_p and B_q: the prologue's, in
+// front of its QK and behind it).  K pair v lies in slot v % 3.  Pair 0 is read
+// between B_p and B_q, pair v > 0 between B_{v-2} and B_{v-1}: in iteration v - 1.
+// Iteration u copies pair u + 3 over pair u, which every wave has read before B_q
+// (u = 0) or B_{u-1}, and each wave waits for those copies before B_{u+1}, after
+// which they are read.  V pair v lies in slot v % 2, is copied in iteration v, waited
+// for before B_v and read in iteration v + 1, over pair v - 2, read before B_{v-1}.
+// So a slot is free only behind the barrier that follows its last read.
+//   The copies are spread over the MFMAs row by row, V of pair u during its PV part,
+// K of pair u+3 during its QK part, and the scalar work (level counts, page addresses) is done between them.  Every
 // sum and every rescale is formed in prefill_kernel's order, so both give the
 // same bits, and chunked prefill those of a single shot.
 //   What bounds it: the LDS operand reads (4 waves x 1 KB per 32-cycle MFMA are
@@ -1087,6 +1095,7 @@ void prefill_solo_kernel(PrefillArgs a) {
     const lds_u8* kb = smem + k_lane;
     qk_blocks(lm, kb, Qf, Cm, S);
   }
+  pf_barrier();  // iteration 0 copies K pair 3 over pair 0
   bf16x8 Pf[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) Pf[i] = bf16x8{};

@@ -306,3 +306,41 @@ def test_prefill_operand_ring_keeps_lds_reads_in_flight(kernel_asm):
         runs = sorted(pipelined_runs(waits), reverse=True)
         assert runs[0] >= 31, (name, runs)
         assert len(runs) >= 2 and runs[1] >= 25, (name, runs)
+
+
+def copies_between_barriers(asm, kernel):
+    """Per stretch between two barriers of `kernel` (in the listing's order): (MFMAs, global->LDS copies)."""
+    start = asm.index(kernel + ":")
+    out = [[0, 0]]
+    for _, s in _instructions(asm[start:asm.index("s_endpgm", start)]):
+        if s.startswith("s_barrier"):
+            out.append([0, 0])
+        out[-1][0] += s.startswith("v_mfma")
+        out[-1][1] += s.startswith("buffer_load") and s.endswith(" lds")
+    return [tuple(x) for x in out]
+
+
+SOLO_KERNELS = tuple(n.replace("14prefill_kernel", "19prefill_solo_kernel") for n in PREFILL_KERNELS)
+
+
+def test_barrier_scanner_counts_copies():
+    asm = """k:
+        buffer_load_dwordx4 v1, s[0:3], 0 offen lds
+        s_barrier
+        v_mfma_f32_32x32x16_bf16 v[0:15], v[16:19], v[20:23], v[0:15]
+        buffer_load_dwordx4 v[4:7], v1, s[0:3], 0 offen
+        s_barrier
+        buffer_load_dwordx4 v1, s[0:3], 0 offen offset:1024 lds
+        s_endpgm
+    """
+    assert copies_between_barriers(asm, "k") == [(0, 1), (1, 0), (0, 1)]
+
+
+def test_first_qk_of_the_128_row_prefill_is_closed_by_a_barrier(kernel_asm):
+    # The prologue's QK reads the K ring's slot 0, and the first iteration copies pair 3 into it: the QK
+    # lies between two barriers, with no copy among its MFMAs.
+    for name in SOLO_KERNELS:
+        before, first_qk, loop = copies_between_barriers(kernel_asm["atf_prefill.hip"], name)[:3]
+        assert before == (0, 24), (name, before)   # K of pairs 0 to 2, two pages of four rows each
+        assert first_qk[0] >= 4 and first_qk[1] == 0, (name, first_qk)
+        assert loop[0] >= 64 and loop[1] >= 16, (name, loop)
