@@ -201,6 +201,11 @@ def _hipcc_or_skip():
     return B
 
 
+def _flags(B, src=None):
+    """The library's flags for `src`, its own ones included, without the resource remarks."""
+    return [f for f in B.COMMON if not f.startswith("-Rpass")] + B.EXTRA.get(os.path.basename(src or ""), [])
+
+
 @pytest.fixture(scope="module")
 def kernel_asm(tmp_path_factory):
     B = _hipcc_or_skip()
@@ -210,8 +215,7 @@ def kernel_asm(tmp_path_factory):
         if not src.endswith(".hip"):
             continue
         dst = os.path.join(tmp, os.path.basename(src) + ".s")
-        flags = [f for f in B.COMMON if not f.startswith("-Rpass")]
-        cmd = [B.HIPCC, *flags, "-I", B.CSRC, "--cuda-device-only", "-S", src, "-o", dst]
+        cmd = [B.HIPCC, *_flags(B, src), "-I", B.CSRC, "--cuda-device-only", "-S", src, "-o", dst]
         p = subprocess.run(cmd, capture_output=True, text=True)
         assert p.returncode == 0, p.stderr
         with open(dst) as f:
@@ -226,12 +230,11 @@ def test_kernel_sources_assemble(tmp_path):
     instruction needs a scalar one) only shows when an object is built: every
     kernel source is assembled to a device object here."""
     B = _hipcc_or_skip()
-    flags = [f for f in B.COMMON if not f.startswith("-Rpass")]
     for src in B.sources():
         if not src.endswith(".hip"):
             continue
         dst = os.path.join(tmp_path, os.path.basename(src) + ".o")
-        p = subprocess.run([B.HIPCC, *flags, "-I", B.CSRC, "--cuda-device-only", "-c", src, "-o", dst],
+        p = subprocess.run([B.HIPCC, *_flags(B, src), "-I", B.CSRC, "--cuda-device-only", "-c", src, "-o", dst],
                            capture_output=True, text=True)
         assert p.returncode == 0, p.stderr[-3000:]
 
@@ -247,7 +250,7 @@ def test_assembling_catches_a_planted_vector_operand(tmp_path):
                    '  asm volatile("s_cmp_le_i32 %0, 1" :: "s"(x) : "scc");\n'
                    '  o[threadIdx.x] = x;\n'
                    '}\n')
-    flags = [f for f in B.COMMON if not f.startswith("-Rpass")]
+    flags = _flags(B)
     listing = subprocess.run([B.HIPCC, *flags, "--cuda-device-only", "-S", str(src), "-o", str(tmp_path / "p.s")],
                              capture_output=True, text=True)
     obj = subprocess.run([B.HIPCC, *flags, "--cuda-device-only", "-c", str(src), "-o", str(tmp_path / "p.o")],
@@ -266,19 +269,37 @@ def test_no_dot_result_hazards(kernel_asm):
         assert dot_hazards(asm) == [], name
 
 
-# the two instantiations of the prefill kernel: scores scaled through Q (RoPE at
+# the two instantiations of each prefill kernel: scores scaled through Q (RoPE at
 # load) and raw scores scaled in the softmax (pre-rotated Q)
 PREFILL_KERNELS = ("_ZN3atf14prefill_kernelILb0EEEvNS_11PrefillArgsE", "_ZN3atf14prefill_kernelILb1EEEvNS_11PrefillArgsE")
+SOLO_KERNELS = tuple(n.replace("14prefill_kernel", "19prefill_solo_kernel") for n in PREFILL_KERNELS)
+
+
+def test_the_listing_is_the_shipped_build(kernel_asm):
+    """Per-file flags reach the listing: the decode kernels preload their scalar arguments, and the 128-row
+    prefill kernel's MFMAs write ordinary registers (without its flag they write accumulation registers)."""
+    assert re.search(r"\.amdhsa_user_sgpr_kernarg_preload_length\s+14", kernel_asm["atf_decode.hip"])
+    asm = kernel_asm["atf_prefill.hip"]
+    for name in SOLO_KERNELS:
+        start = asm.index(name + ":")
+        mfma = [s for _, s in _instructions(asm[start:asm.index("s_endpgm", start)]) if s.startswith("v_mfma")]
+        assert len(mfma) > 64 and all(re.match(r"\S+\s+v\[", s) for s in mfma), name
 
 
 def test_prefill_kernel_does_not_spill(kernel_asm):
     asm = kernel_asm["atf_prefill.hip"]
     # kernel metadata: one "- .agpr_count" block per kernel, holding .name and .vgpr_spill_count
-    for name in PREFILL_KERNELS:
+    for name in PREFILL_KERNELS + SOLO_KERNELS:
         blocks = [b for b in asm.split("  - .agpr_count:") if re.search(r"\.name:\s+" + name + r"\s", b)]
         assert len(blocks) == 1, f"{name} metadata not found"
         spill = re.search(r"\.vgpr_spill_count:\s+(\d+)", blocks[0])
         assert spill and int(spill.group(1)) == 0, name
+
+
+def test_decode_and_writer_kernels_do_not_spill(kernel_asm):
+    for src, least in (("atf_decode.hip", 16), ("atf_kv_write.hip", 4)):
+        spills = re.findall(r"\.vgpr_spill_count:\s+(\d+)", kernel_asm[src])
+        assert len(spills) >= least and set(spills) == {"0"}, (src, spills)
 
 
 def pipelined_runs(waits, depth=3):
@@ -300,7 +321,7 @@ def test_prefill_operand_ring_keeps_lds_reads_in_flight(kernel_asm):
     # the PV stream of a tile pair (32 MFMAs) and the 8-level QK stream of its
     # four 32-key blocks (32 MFMAs, the ring draining over the last three) run
     # with the operand reads of several later MFMAs still outstanding
-    for name in PREFILL_KERNELS:
+    for name in PREFILL_KERNELS + SOLO_KERNELS:
         waits = lds_waits_before_mfma(kernel_asm["atf_prefill.hip"], name)
         assert len(waits) >= 64, name
         runs = sorted(pipelined_runs(waits), reverse=True)
@@ -318,9 +339,6 @@ def copies_between_barriers(asm, kernel):
         out[-1][0] += s.startswith("v_mfma")
         out[-1][1] += s.startswith("buffer_load") and s.endswith(" lds")
     return [tuple(x) for x in out]
-
-
-SOLO_KERNELS = tuple(n.replace("14prefill_kernel", "19prefill_solo_kernel") for n in PREFILL_KERNELS)
 
 
 def test_barrier_scanner_counts_copies():
