@@ -25,21 +25,24 @@ namespace atf {
 // outside the call keep their contents.  Tokens at negative positions, past
 // max_pages, past the RoPE table or whose page-table entry is invalid are
 // skipped, as one token at a time would be.
-//   HBM bound: 16K tokens x 8 heads 35.9 us a call with one workgroup looping
-// over all heads of a page (8 waves a CU), 26.1 with one per four heads
-// (142 MB: 5.5 TB/s); 64K x 4 heads 58.7 us.
-// grid: x = page index relative to the call's first page, y = sequence, z = heads
-// kHeads z .. kHeads z + kHeads - 1.
-template <int kHeads>
+//   HBM bound: see launch_kv_write.
+// kHeadsFirst: grid x = heads, y = page index relative to the call's first page, z =
+// sequence, so that the workgroups of a page run together and its (cos, sin) rows
+// are read from memory once; the heads turn every eight pages, so that no XCD
+// writes the same ones throughout (30000 x 8: 55.6 us a call, 58.4 without).
+// Otherwise x = page, y = sequence, z = heads.
+template <int kHeads, bool kHeadsFirst>
 __global__ __launch_bounds__(128) void kv_write_kernel(KvWriteArgs a) {
   __shared__ __attribute__((aligned(16))) uint16_t sv[kHeads][kPage][kD];
-  const int b = blockIdx.y;
-  const int h0 = blockIdx.z * kHeads;
+  const int b = kHeadsFirst ? blockIdx.z : blockIdx.y;
+  const int per = kHeadsFirst ? (a.hkv + gridDim.x - 1) / gridDim.x : kHeads;  // heads of a workgroup, at most kHeads
+  const int h0 = (kHeadsFirst ? (blockIdx.x + blockIdx.y / 8) % gridDim.x : blockIdx.z) * per;
+  const int h_end = min(a.hkv, h0 + per);
   const int tid = threadIdx.x;
   const int start = a.start_pos[b];
   const int64_t end64 = static_cast<int64_t>(start) + a.n_tokens;  // exclusive
   const int first = max(start, 0) >> 4;
-  const int pidx = first + static_cast<int>(blockIdx.x);
+  const int pidx = first + static_cast<int>(kHeadsFirst ? blockIdx.y : blockIdx.x);
   const int64_t p0 = static_cast<int64_t>(pidx) * kPage;
   if (pidx >= a.max_pages || p0 >= end64) return;
   // covered slots [s0, s1) of this page
@@ -67,14 +70,14 @@ __global__ __launch_bounds__(128) void kv_write_kernel(KvWriteArgs a) {
     u32x4 x1[kHeads], x2[kHeads];
 #pragma unroll
     for (int j = 0; j < kHeads; ++j) {
-      if (h0 + j < a.hkv) {
+      if (h0 + j < h_end) {
         x1[j] = ldg16(krow + static_cast<int64_t>(h0 + j) * a.ks_h + c0);
         x2[j] = ldg16(krow + static_cast<int64_t>(h0 + j) * a.ks_h + c1);
       }
     }
 #pragma unroll
     for (int j = 0; j < kHeads; ++j) {
-      if (h0 + j < a.hkv) {
+      if (h0 + j < h_end) {
         u32x4 y1 = x1[j], y2 = x2[j];
         if (a.rope_cs != nullptr) {
           y1 = rope_half(x1[j], x2[j], cs, false);
@@ -103,7 +106,7 @@ __global__ __launch_bounds__(128) void kv_write_kernel(KvWriteArgs a) {
     for (int r = 0; r < 2; ++r) {
       const int idx = tid + 128 * r;  // token idx/16, 16-byte chunk idx%16
       const int tok = idx >> 4, ch = idx & 15;
-      if (h0 + j < a.hkv && tok >= s0 && tok < s1) {
+      if (h0 + j < h_end && tok >= s0 && tok < s1) {
         const uint16_t* vrow = a.v_src + static_cast<int64_t>(b) * a.vs_b +
                                static_cast<int64_t>(t0 + tok) * a.vs_t + static_cast<int64_t>(h0 + j) * a.vs_h;
         *reinterpret_cast<u32x4*>(&sv[j][tok][8 * ch]) = ldg16(vrow + 8 * ch);
@@ -114,7 +117,7 @@ __global__ __launch_bounds__(128) void kv_write_kernel(KvWriteArgs a) {
   const int d = tid;
 #pragma unroll
   for (int j = 0; j < kHeads; ++j) {
-    if (h0 + j >= a.hkv) break;
+    if (h0 + j >= h_end) break;
     uint16_t* vdst = a.kv_cache + blk0 + static_cast<size_t>(h0 + j) * kKvBlockElems + d * kPage;
     uint32_t w[8];  // the row's 16 slots as 8 packed pairs
     if (s0 == 0 && s1 == kPage) {
@@ -187,6 +190,21 @@ __global__ __launch_bounds__(128) void kv_append_kernel(KvWriteArgs a) {
   }
 }
 
+// kv_write_kernel with at most kHeads heads a workgroup.  The heads come first in
+// the grid for calls of more than 128K token x head rows (24000 x 8: 45.7 us a call,
+// 46.8 with the heads last; 12000 x 16 45, 50; below, 8192 x 8: 19.6, 19.4) whose
+// heads divide evenly (otherwise every second workgroup, and with it every second
+// XCD, would have the lighter share).
+template <int kHeads>
+static void launch_pages(const KvWriteArgs& a, int pages, int64_t rows, hipStream_t s) {
+  const int groups = (a.hkv + kHeads - 1) / kHeads;
+  const bool even = groups > 1 && rows > 128 * 1024 && a.hkv % groups == 0 && pages <= 65535 && a.batch <= 65535;
+  if (even)
+    hipLaunchKernelGGL((kv_write_kernel<kHeads, true>), dim3(groups, pages, a.batch), dim3(128), 0, s, a);
+  else
+    hipLaunchKernelGGL((kv_write_kernel<kHeads, false>), dim3(pages, a.batch, groups), dim3(128), 0, s, a);
+}
+
 hipError_t launch_kv_write(const KvWriteArgs& a, hipStream_t s) {
   if (a.n_tokens <= 0 || a.batch <= 0) return hipSuccess;
   if (a.n_tokens <= kKvAppendTokens && a.hkv <= 65535 && a.batch <= 65535) {
@@ -196,16 +214,19 @@ hipError_t launch_kv_write(const KvWriteArgs& a, hipStream_t s) {
   // a call of n tokens touches at most ceil(n / 16) + 1 pages per sequence
   const int pages = (a.n_tokens + kPage - 1) / kPage + 1;
   // Heads per workgroup, by the call's token x head rows: few rows are spread over
-  // more workgroups (517 tokens x 4 heads: kernel 8.1 us with four heads, 5.6 two,
-  // 4.8 one; calls on fresh buffers: 8192 x 8 17.0, 15.8, 17.2; 16K x 8 33.6,
-  // 33.0, 35.0); many share the (cos, sin) rows (128K x 4: 115.9, 123.3, 133.0).
+  // more workgroups, many share the (cos, sin) rows.  us a call with one, two and
+  // four heads (three sources and caches in turn): 1000 x 8 5.2, 6.3, 8.8; 4000 x 8
+  // 10.7, 10.6, 13.2; 16K x 8 36.1, 33.8, 34.5; 3 x 20000 x 8 115, 102, 105; 64K x 8
+  // 126, 113, 113; 128K x 8 247, 218, 214; 64K x 4 64.9, 59.3, 61.0; 128K x 4 125, 117 to
+  // 120, 117.  An odd head count leaves two heads a workgroup uneven: 64K x 5 82, 77, 75.
+  // One workgroup looping over all heads of a page takes 36.3 at 16K x 8 and 221 at
+  // 128K x 8; with the heads in the z dimension the (cos, sin) rows of a long call are
+  // read again for each group: 128K x 8 231 and not 214, 128K x 16 467 and not 401.
   const int64_t rows = static_cast<int64_t>(a.n_tokens) * a.batch * a.hkv;
-  if (rows <= 32 * 1024 || a.hkv == 1)
-    hipLaunchKernelGGL(kv_write_kernel<1>, dim3(pages, a.batch, a.hkv), dim3(128), 0, s, a);
-  else if (rows < 256 * 1024 || a.hkv == 2)
-    hipLaunchKernelGGL(kv_write_kernel<2>, dim3(pages, a.batch, (a.hkv + 1) / 2), dim3(128), 0, s, a);
-  else
-    hipLaunchKernelGGL(kv_write_kernel<4>, dim3(pages, a.batch, (a.hkv + 3) / 4), dim3(128), 0, s, a);
+  const int64_t four = (a.hkv % 2 == 0 ? 512 : 256) * 1024;
+  if (rows <= 32 * 1024 || a.hkv == 1) launch_pages<1>(a, pages, rows, s);
+  else if (rows < four || a.hkv == 2) launch_pages<2>(a, pages, rows, s);
+  else launch_pages<4>(a, pages, rows, s);
   return hipGetLastError();
 }
 

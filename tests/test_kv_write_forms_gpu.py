@@ -37,7 +37,9 @@ def test_few_tokens(n, hkv, start, layout, dev):
         assert torch.equal(kv.cpu(), _assemble(ek, ev)), table
 
 
-@pytest.mark.parametrize("B,n,hkv", [(1, 300, 1), (2, 3000, 7), (1, 5000, 9), (3, 9000, 5), (1, 70001, 2), (1, 15000, 9)])
+# (rows of tokens x heads at and past each line; heads that divide evenly come first in the grid, others last)
+@pytest.mark.parametrize("B,n,hkv", [(1, 300, 1), (2, 3000, 7), (1, 5000, 9), (3, 9000, 5), (1, 70001, 2), (1, 15000, 9),
+                                     (2, 5000, 4), (3, 4111, 6), (1, 65536, 8), (2, 43700, 6), (1, 33000, 16)])
 def test_forms_agree(B, n, hkv, dev):
     """A call by the two- or four-head kernel (odd head counts: a last group
     partly empty) equals calls of 100 tokens (one head per workgroup) and of 3
