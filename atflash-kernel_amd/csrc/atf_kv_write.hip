@@ -194,12 +194,13 @@ __global__ __launch_bounds__(128) void kv_append_kernel(KvWriteArgs a) {
 // the grid for calls of more than 128K token x head rows (24000 x 8: 45.7 us a call,
 // 46.8 with the heads last; 12000 x 16 45, 50; below, 8192 x 8: 19.6, 19.4) whose
 // heads divide evenly (otherwise every second workgroup, and with it every second
-// XCD, would have the lighter share).
+// XCD, would have the lighter share) and, whatever they are, where they would not
+// fit the z dimension.
 template <int kHeads>
 static void launch_pages(const KvWriteArgs& a, int pages, int64_t rows, hipStream_t s) {
   const int groups = (a.hkv + kHeads - 1) / kHeads;
   const bool even = groups > 1 && rows > 128 * 1024 && a.hkv % groups == 0 && pages <= 65535 && a.batch <= 65535;
-  if (even)
+  if (groups > 65535 || even)
     hipLaunchKernelGGL((kv_write_kernel<kHeads, true>), dim3(groups, pages, a.batch), dim3(128), 0, s, a);
   else
     hipLaunchKernelGGL((kv_write_kernel<kHeads, false>), dim3(pages, a.batch, groups), dim3(128), 0, s, a);

@@ -61,3 +61,20 @@ def test_forms_agree(B, n, hkv, dev):
         ops.kv_write(parts, k[:, t:t + step], v[:, t:t + step], starts + t, table, rt, 0)
         t += step
     assert torch.equal(whole, parts)
+
+
+@pytest.mark.parametrize("n,hkv", [(2, 65536), (1, 131080), (1, 131081)])
+def test_many_heads(n, hkv, dev):
+    """More heads, and more pairs of heads, than a grid's y and z dimensions hold; tokens at the end of one
+    page and the start of the next."""
+    print(f"[kv_write heads] n={n} hkv={hkv}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(hkv)
+    k, v = (torch.randn((1, n, hkv, H.D), generator=g, device=dev).to(torch.bfloat16) for _ in range(2))
+    kv = torch.zeros((2, hkv, 2, 2048), dtype=torch.bfloat16, device=dev)
+    ops.kv_write(kv, k, v, torch.tensor([15], dtype=torch.int32, device=dev),
+                 torch.tensor([[1, 0]], dtype=torch.int32, device=dev), None, 1)
+    want = torch.zeros_like(kv)
+    for t, (page, slot, v_slot) in enumerate([(1, 15, 15), (0, 0, 0)][:n]):
+        want[page, :, 0].view(hkv, 128, 16)[:, :, v_slot] = v[0, t]
+        want[page, :, 1].view(hkv, 16, 16, 8)[:, :, slot] = k[0, t].view(hkv, 16, 8)
+    assert torch.equal(kv, want)
