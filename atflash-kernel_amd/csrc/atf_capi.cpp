@@ -247,7 +247,6 @@ int atf_prefill_bf16(void* out, int64_t o_sb, int64_t o_st, int64_t o_sh, float*
   a.hq = num_q_heads;
   a.hkv = num_kv_heads;
   a.group = num_q_heads / num_kv_heads;
-  a.n_qtiles = (nq + atf::kPfRowsWg - 1) / atf::kPfRowsWg;
   a.sm_scale = sm_scale;
   a.scale_log2 = sm_scale * 1.4426950408889634f;
   a.rope_cs = rope_cs;

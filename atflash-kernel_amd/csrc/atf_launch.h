@@ -51,7 +51,7 @@ struct PrefillArgs {
   const int32_t* page_table;
   int max_pages;
   int batch, nq, nk, q_offset, hq, hkv, group;
-  int n_qtiles;
+  int n_qtiles;  // set by launch_prefill for the kernel it picks
   float scale_log2;
   float sm_scale;
   const float* rope_cs;

@@ -395,32 +395,6 @@ __device__ __forceinline__ void qk_stream(const lds_u8* kb, bf16x8 (&f)[kRing], 
   }
 }
 
-// The MFMA phase of tile pair u with one level count L for its four 32-key
-// blocks: PV of the previous pair, then QK of this pair, as one straight-line
-// stream (the level counts are known before the phase starts, so nothing
-// branches between its first LDS read and its last MFMA).
-template <int L>
-__device__ __forceinline__ void mfma_phase(const lds_u8* vb, const lds_u8* kb, const bf16x8 (&Pf)[8],
-                                           f32x16 (&O)[4], const u32x4 (&Qf)[kLevels], const f32x16& C,
-                                           f32x16 (&S)[4]) {
-  bf16x8 f[kRing];
-  pv_prefetch(vb, f);
-  pv_stream(vb, kb, Pf, O, f);
-  qk_stream<L>(kb, f, Qf, C, S);
-}
-
-// The MFMA phase of a pair with a level boundary inside it (L0 <= L1 <= L2 <= L3,
-// not all equal): PV as above, then per-tile chains.
-__device__ __forceinline__ void mfma_phase_mixed(int L0, int L1, int L2, int L3, const lds_u8* vb,
-                                                 const lds_u8* kb, const bf16x8 (&Pf)[8], f32x16 (&O)[4],
-                                                 const u32x4 (&Qf)[kLevels], const f32x16& C, f32x16 (&S)[4]) {
-  bf16x8 f[kRing];
-  pv_prefetch(vb, f);
-  pv_stream(vb, kb, Pf, O, f);
-  qk_tile(L0, L1, kb, kb + 8192, Qf, f[32 % kRing], f[33 % kRing], C, S[0], S[1]);
-  qk_tile(L2, L3, kb + 16384, kb + 24576, Qf, f[34 % kRing], f[35 % kRing], C, S[2], S[3]);
-}
-
 // P = exp2(S) of one 32-key block (S[kb]) packed to bf16 (Pf[2kb], Pf[2kb+1]
 // are the B operands of the PV steps of its two pages), added to the lane's
 // partial row sum lt.  kRaw: S is in raw score units (Q was not scaled) and
@@ -462,7 +436,8 @@ __device__ __forceinline__ float exp_tiles(const f32x16 (&S)[4], bf16x8 (&Pf)[8]
 //   24 / 8 heads, OFF: 8 x 700 tokens 81.5 -> 66 us, 8 x 256 26 -> 20, 64 x 256
 // 152 -> 121; 28 / 4 heads, k = 2: 2048 tokens 56.5 -> 51, 4096 128 -> 120, 32768
 // 5.22 -> 5.16 ms; 128 tokens 13.6 -> 10.9.  A launch of one or two waves pays the
-// LDS round trips instead: up to 32 tokens 11.1 -> 11.7.
+// LDS round trips instead, 0.6 us of 11.7 up to 32 tokens (13.6 to 14.1 in the
+// 256-row kernel with fragment loads).
 constexpr int kRowStage = 32 * 2 * kP * 2;           // 32 rows, 8 KB a wave
 typedef u32x4 u32x4_a8 __attribute__((aligned(8)));    // `out` is 8-byte aligned
 
