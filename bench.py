@@ -2,9 +2,9 @@
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--n 131072] [--no-cpu-baseline]
 
-Workload (BASELINE.json metric "prefill ms + decode us/step @128K, Qwen2.5-7B
-shape, window ON vs OFF; %roofline"): Hq = 28, Hkv = 4, d = 128, RoPE base 1e7,
-bf16 N(0,1) synthetic tensors from a fixed seed.
+Workload (prefill ms + decode us/step @128K, Qwen2.5-7B shape, window ON vs OFF;
+%roofline): Hq = 28, Hkv = 4, d = 128, RoPE base 1e7, bf16 N(0,1) synthetic
+tensors from a fixed seed.
   prefill  one causal GQA prefill over N = 128K tokens: the full op
            (K RoPE + paged-cache pack, then the attention kernel with Q RoPE at
            load), for window OFF, k = 2 and k = 64;
@@ -21,8 +21,9 @@ stream, with device synchronisation around the timed region.  Decode is also
 timed as back-to-back launches under one event pair per batch of 8*K (the
 median of five batches); that per-launch average (no event packets between
 launches) is the decode figure in `detail` and `roofline_decode`.
-`value` is the window-ON (k = 2) prefill time in ms (lower is better); every
-configuration's numbers are in `detail`.
+`value` is the window-ON (k = 2) prefill time in ms (lower is better).  The result
+is the last line, with a few of the other numbers in its `detail`; the whole of
+`detail` is a line before it, behind "[bench detail json] ".
 roofline  prefill attention kernel (MFMA bound): algorithmic FLOPs per launch
           (2*Hq*N^2*d window OFF; Hq*N^2*d*(1+s) window ON, s = QK slice ratio
           at the kernel's (32, 32) tiles) / mean kernel time, against 2.5 PFLOP/s;
@@ -181,6 +182,9 @@ class ClockSampler:
             if d_acc > 0:
                 out["ppt_residency"] = (self.last["ppt"] - self.first["ppt"]) / d_acc
         return out
+
+
+DETAIL_PREFIX = "[bench detail json] "
 
 
 def _traffic():
@@ -968,34 +972,39 @@ def main():
                               "frac": kvw["frac"], "traffic": kvw["traffic"], "bytes": kvw_bytes,
                               "kernel": f"atf::kv_write_kernel, {N} tokens x {HKV} kv heads",
                               "us_per_launch": kvw["us_per_launch"]},
-        "detail": {
-            "prefill_ms": {n: pre[n]["median_ms"] for n in pre},
-            "prefill_attn_kernel_ms": {n: attn[n]["median_ms"] for n in attn},
-            "decode_us": {n: res["decode"][n]["batch_mean_ms"] * 1e3 for n in res["decode"]},
-            "decode_us_per_call_median": {n: res["decode"][n]["median_ms"] * 1e3 for n in res["decode"]},
-            "decode_us_graph": {n: res["decode"][n]["graph_mean_ms"] * 1e3 for n in res["decode"]},
-            "prefill_on_over_off": {n: pre["off"]["median_ms"] / pre[n]["median_ms"] for n in ("k2", "k64")},
-            "decode_on_over_off": {n: res["decode"]["off"]["batch_mean_ms"] / res["decode"][n]["batch_mean_ms"]
-                                   for n in res["decode"] if n != "off"},
-            "decode_on_over_off_graph": {n: res["decode"]["off"]["graph_mean_ms"] / res["decode"][n]["graph_mean_ms"]
-                                         for n in res["decode"] if n != "off"},
-            "clocks": res["clocks"],
-            "slice_ratios": sr,
-            "ceilings": {n: {"prefill": 2 / (1 + sr[n]["s_prefill"]), "decode": 2 / (1 + sr[n]["s_decode"]),
-                             "decode_vec8": 2 / (1 + sr[n]["s_decode_vec8"])} for n in sr},
-            "kv_write_us": kvw["us_per_launch"],
-            "decode_pool_bytes": res["decode_pool_bytes"],
-            "timed_region_wall_s": wall,
-            "stats": {k: v for k, v in res.items() if k != "clocks"},
-        },
+    }
+    detail = {
+        "prefill_ms": {n: pre[n]["median_ms"] for n in pre},
+        "prefill_attn_kernel_ms": {n: attn[n]["median_ms"] for n in attn},
+        "decode_us": {n: res["decode"][n]["batch_mean_ms"] * 1e3 for n in res["decode"]},
+        "decode_us_per_call_median": {n: res["decode"][n]["median_ms"] * 1e3 for n in res["decode"]},
+        "decode_us_graph": {n: res["decode"][n]["graph_mean_ms"] * 1e3 for n in res["decode"]},
+        "prefill_on_over_off": {n: pre["off"]["median_ms"] / pre[n]["median_ms"] for n in ("k2", "k64")},
+        "decode_on_over_off": {n: res["decode"]["off"]["batch_mean_ms"] / res["decode"][n]["batch_mean_ms"]
+                               for n in res["decode"] if n != "off"},
+        "decode_on_over_off_graph": {n: res["decode"]["off"]["graph_mean_ms"] / res["decode"][n]["graph_mean_ms"]
+                                     for n in res["decode"] if n != "off"},
+        "clocks": res["clocks"],
+        "slice_ratios": sr,
+        "ceilings": {n: {"prefill": 2 / (1 + sr[n]["s_prefill"]), "decode": 2 / (1 + sr[n]["s_decode"]),
+                         "decode_vec8": 2 / (1 + sr[n]["s_decode_vec8"])} for n in sr},
+        "kv_write_us": kvw["us_per_launch"],
+        "decode_pool_bytes": res["decode_pool_bytes"],
+        "timed_region_wall_s": wall,
+        "stats": {k: v for k, v in res.items() if k != "clocks"},
     }
     if detail_cfgs is not None:
-        line["detail"]["configs"] = detail_cfgs
+        detail["configs"] = detail_cfgs
     if c5 is not None:
-        line["detail"]["configs"]["c5"] = c5
+        detail["configs"]["c5"] = c5
     if not args.no_cpu_baseline:
         line["cpu_baseline"] = cpu_baseline(N)
-    print(json.dumps(line))
+    # The measurements behind the result, on a line of their own: the result line, the last one, stays short
+    # enough for a reader of the output's end.
+    print(DETAIL_PREFIX + json.dumps(detail))
+    line["detail"] = {k: detail[k] for k in ("prefill_ms", "decode_us", "prefill_on_over_off", "decode_on_over_off",
+                                             "decode_on_over_off_graph", "kv_write_us")}
+    print(json.dumps(line), flush=True)
 
 
 if __name__ == "__main__":
