@@ -948,10 +948,11 @@ __device__ __forceinline__ void qk_blocks(uint64_t lm, const lds_u8* kb, const u
 // K of pair u+3 during its QK part, and the scalar work (level counts, page addresses) is done between them.  Every
 // sum and every rescale is formed in prefill_kernel's order, so both give the
 // same bits, and chunked prefill those of a single shot.
-//   What bounds it: the LDS operand reads (4 waves x 1 KB per 32-cycle MFMA are
-// the LDS' 128 bytes a clock) and, in the PV part, one wave's issue of 32 MFMAs,
-// 64 exps, 64 adds and 32 packings (about 60 cycles an MFMA).  1024 queries behind
-// 32K keys, 28 / 4 heads: k = 2 531 -> 431 us, OFF 602 -> 472; 517 tokens 29 -> 20; where the chip is
+//   What bounds it: one wave's own chain, in the PV part the issue of 32 MFMAs, 64
+// exps, 64 adds and 32 packings (about 60 cycles an MFMA), with no other wave on the
+// SIMD to fill it.  1024 queries behind 32K keys, 28 / 4 heads, k = 2: the matrix pipes
+// are busy 43% of the time of the CUs in use, the LDS index unit 22%, 1% of that in
+// conflicts.  There k = 2 531 -> 431 us, OFF 602 -> 472; 517 tokens 29 -> 20; where the chip is
 // full it loses (4096 tokens 127 -> 152 us), a pair taking 3100 to 3500 cycles for
 // 32 rows of a SIMD where prefill_kernel takes 5000 to 5700 for 64.
 constexpr int kSoloWaves = 4;

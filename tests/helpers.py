@@ -8,8 +8,8 @@ from oracle import window_rule as WR
 
 D = 128
 BF = torch.bfloat16
-TOL_MAX = 2e-2   # max |out - fp32 oracle|
-TOL_MEAN = 1e-3  # mean |out - fp32 oracle|
+TOL_MAX = 2e-2   # accuracy bar: max |out - fp32 oracle|
+TOL_MEAN = 1e-3  # accuracy bar: mean |out - fp32 oracle|
 PREFILL_BM, PREFILL_BN, DECODE_BN = 32, 32, 16
 
 

@@ -84,7 +84,7 @@ def test_prefill_query_offset_matches_oracle(q_offset, nq, k_ret, dev):
 
 def test_prefill_llama_shape_reports_bf16_anchor(dev):
     """Llama-3.2-3B shape at the reference's correctness seed (777,
-    microbench/b1_correctness.py:218): the pass criterion is the north-star bar
+    microbench/b1_correctness.py:218): the pass criterion is the accuracy bar
     against the fp32 oracle.  The reference's own rule,
     max err <= 2 * max|ref16 - ref32| + 2e-3, is printed for comparison only:
     its bf16 anchor (torch CPU bf16 matmuls) is not pinned bit for bit here, so

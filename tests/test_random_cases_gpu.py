@@ -1,5 +1,5 @@
 """Seeded random parity sweep (GPU): shapes, windows and layouts drawn from a
-fixed generator, each checked against the fp32 oracle at the north-star bar.
+fixed generator, each checked against the fp32 oracle at the accuracy bar.
 
 Prefill: batch 1-2, GQA group 1-8, 1-4 kv heads, up to 1200 keys, a query
 chunk of any length at the bottom-right end (offsets not multiples of the
